@@ -47,9 +47,8 @@ enum {
     KAM_TRANSFORM_FFT = 0,  /* the row FFT in LDS (default) */
     KAM_TRANSFORM_DFT = 1,  /* dense DFT products on MFMA: FP16 hi/lo operands, FP32
                                accumulate (FP32-pressure simulations, n_theta <= 1024) */
-    KAM_TRANSFORM_FFT8 = 2  /* the row FFT with a forward kernel that stages half the
-                               twiddle table and runs eight waves per SIMD; a batch takes
-                               it when all its FFT simulations do.  Same values as FFT. */
+    KAM_TRANSFORM_FFT8 = 2  /* as KAM_TRANSFORM_FFT (the name of an earlier eight-wave
+                               forward kernel, still accepted).  Same values. */
 };
 
 /* ---- precision modes ----------------------------------------------------- */
@@ -356,8 +355,8 @@ int kam_tune_set_transform(int n_theta, int transform);
 int kam_tune_get_transform(int n_theta, int *transform);
 
 /* Times candidate shapes on `batch` synthetic simulations of n_theta (steps
- * timed steps each): advection tiles, FFT tile heights, then the two row FFT
- * forms against each other and against the MFMA DFT (n_theta <= 1024).  Records the fastest with
+ * timed steps each): advection tiles, FFT tile heights, then the row FFT
+ * against the MFMA DFT (n_theta <= 1024).  Records the fastest with
  * kam_tune_set and kam_tune_set_transform, appends a line
  * "gfx950 n_theta batch adv_rows adv_cols fft_rows adv_ms fft_ms transform"
  * to cache_path (may be NULL), and returns the best per-kernel times in

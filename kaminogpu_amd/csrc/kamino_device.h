@@ -57,6 +57,41 @@ enum SimFlags {
     SIM_DFT = 4   // phi transforms as dense DFTs on MFMA (FP16 hi/lo matrices) instead of FFTs
 };
 
+// One pass of the row FFT: a radix-R butterfly, or two elementary radices R1
+// and R2 in a row (R = R1 R2) whose values stay in a lane's registers between
+// them, on I items per lane.  A row's passes use the kinds in rising order, so
+// the transform walks this list once instead of branching to each pass (four
+// groups G of kinds are skipped as a whole; a taken branch costs a lone
+// wavefront some 40 cycles, and a switch took about 15 of them per pass).
+#define KAM_FFT_KINDS(X)                                                                     \
+    X(1, 0, 4, 1, 4) X(2, 0, 4, 1, 2) X(3, 0, 4, 1, 1) X(4, 0, 4, 4, 1) X(5, 0, 4, 3, 1)     \
+    X(6, 1, 4, 2, 2) X(7, 1, 4, 2, 1) X(8, 1, 2, 1, 4) X(9, 1, 2, 1, 2) X(10, 1, 2, 1, 1)    \
+    X(11, 1, 2, 3, 2) X(12, 1, 2, 3, 1) X(13, 1, 2, 5, 1)                                    \
+    X(14, 2, 3, 1, 4) X(15, 2, 3, 1, 2) X(16, 2, 3, 1, 1) X(17, 2, 3, 3, 1) X(18, 2, 3, 5, 1) \
+    X(19, 3, 5, 1, 2) X(20, 3, 5, 1, 1)
+constexpr int kFftMaxPass = 8;
+struct alignas(16) FftPass {
+    uint16_t kind, nb;  // nb = M / R items
+    uint16_t Ls, tw0;   // Ls = product of the radices before; tw0 = its first twiddle in the pass table
+    unsigned magic;     // b / Ls == umulhi(b, magic) + (b & unit) for b < 2^16:
+    unsigned unit;      // ceil(2^32 / Ls) and 0, or for Ls = 1 (2^32 does not fit) 0 and ~0
+};
+
+// Rows of 2^k values, 32 <= M <= 2048, have a plan known at compile time, and
+// launches of one such size transform kernels built for it: every address is
+// then a lane's base plus a constant, and a radix-4 pass issues about 60
+// instructions instead of 160 (a lone wavefront pays ~5 cycles for each).  The
+// lists hold R1 R2 of each pass (4, or 8 and 16 as 4 x 2 and 4 x 4).
+template <int M> struct FftPow2;
+template <> struct FftPow2<32> { static constexpr int lanes = 8, n = 2, R[4] = {4, 8}; };
+template <> struct FftPow2<64> { static constexpr int lanes = 16, n = 3, R[4] = {4, 4, 4}; };
+template <> struct FftPow2<128> { static constexpr int lanes = 32, n = 3, R[4] = {4, 4, 8}; };
+template <> struct FftPow2<256> { static constexpr int lanes = 64, n = 4, R[4] = {4, 4, 4, 4}; };
+template <> struct FftPow2<512> { static constexpr int lanes = 64, n = 3, R[4] = {4, 16, 8}; };
+template <> struct FftPow2<1024> { static constexpr int lanes = 64, n = 3, R[4] = {4, 16, 16}; };
+template <> struct FftPow2<2048> { static constexpr int lanes = 128, n = 3, R[4] = {16, 16, 8}; };
+#define KAM_FFT_POW2(X) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048)
+
 struct SimDesc {
     int nTheta, nPhi, M;   // M = nPhi / 2
     int flags;             // SimFlags
@@ -67,13 +102,12 @@ struct SimDesc {
     float* spec;           // float2 M x nTheta4, row-blocked (spec_index)
     const float* rowf;     // RT_COUNT * nTheta
     const double* rowd;    // RD_COUNT * nTheta
-    const float* twN;      // float2 [nPhi]: exp(-2 pi i n / nPhi)
+    const float* twN;      // float2 [nPhi]: w(n) = exp(-2 pi i n / nPhi), n < M, then the M - 1 twiddles
+                           // of the row FFT's passes in the order they are read
     const double* twN64;   // double2 [nPhi]: the same in FP64 (the FP64 pressure transform)
     double invH64;         // 1 / h in FP64
-    int nfac;              // radix factors of M, innermost first
-    int fac[12];
-    int twStep[12];        // per pass p: twiddle index stride nPhi / (Ls r), Ls = fac[0] ... fac[p-1]
-    unsigned lsMagic[12];  // per pass p: ceil(2^32 / Ls) (0 when Ls is a power of two)
+    FftPass pass[kFftMaxPass + 1];  // the row FFT's passes, then kind 0
+    unsigned passKinds;    // bit k: a pass of kind k
     int fftShift;          // log2 of the lanes per row of the row FFT
     int advRows;           // rows per advection tile
     int fftRows;           // rows per FFT tile

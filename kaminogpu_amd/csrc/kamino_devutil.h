@@ -31,6 +31,10 @@ __device__ __forceinline__ float4 ldf4(Rsrc r, int elem) {
 __device__ __forceinline__ void stf(Rsrc r, int vbytes, int sbytes, float v) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, vbytes, sbytes, 0);
 }
+__device__ __forceinline__ void stf2(Rsrc r, int elem, float2 v) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, elem * 4, 0, 0);
+}
 __device__ __forceinline__ float lerpf(float a, float b, float t) { return fmaf(t, b - a, a); }
 
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.

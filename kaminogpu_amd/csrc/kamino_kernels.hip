@@ -783,17 +783,50 @@ __global__ __launch_bounds__(256) void k_particles(const SimDesc* __restrict__ s
 }
 
 // ---------------------------------------------------------------------------
-// Row FFT, one wavefront per row: Stockham autosort passes (radix 2/3/4/5)
-// ping-pong between the row and the wavefront's own scratch row in LDS.  LDS
-// operations of one wavefront complete in issue order, so consecutive passes
-// are separated by a wavefront-scope fence only, never a workgroup barrier.
-// DIR = -1 for exp(-i ...), +1 for exp(+i ...); unnormalised.
+// Row FFT: Stockham autosort passes (radix 2/3/4/5, one or two to a pass) on a
+// row in LDS, in place: a pass reads all its values into registers before it
+// writes any.  DIR = -1 for exp(-i ...), +1 for exp(+i ...); unnormalised.
 // ---------------------------------------------------------------------------
 // Complex arithmetic on float2 (FP32 transforms) and double2 (the FP64
 // pressure transform); R is the component type.
 template <typename C> struct CplxT;
-template <> struct CplxT<float2> { typedef float R; };
-template <> struct CplxT<double2> { typedef double R; };
+template <> struct CplxT<float2> {
+    typedef float R;
+    typedef float V __attribute__((ext_vector_type(2)));
+};
+template <> struct CplxT<double2> {
+    typedef double R;
+    typedef double V __attribute__((ext_vector_type(2)));
+};
+// LDS byte addresses: a pass of runtime size walks them with one addition per
+// access (as array indices, each access costs a multiplication, a shift and an
+// addition, and a lone wavefront pays ~5 cycles for every instruction).  The
+// empty asm keeps the compiler from turning the walk back into products.
+template <typename C>
+__device__ __forceinline__ unsigned lds_addr(const C* p) {
+    return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+template <typename C>
+__device__ __forceinline__ C lds_get(unsigned a) {
+    typedef typename CplxT<C>::V V;
+    const V v = *(const __attribute__((address_space(3))) V*)(uintptr_t)a;
+    C c;
+    c.x = v.x;
+    c.y = v.y;
+    return c;
+}
+template <typename C>
+__device__ __forceinline__ void lds_put(unsigned a, C c) {
+    typedef typename CplxT<C>::V V;
+    V v;
+    v.x = c.x;
+    v.y = c.y;
+    *(__attribute__((address_space(3))) V*)(uintptr_t)a = v;
+}
+__device__ __forceinline__ void lds_step(unsigned& a, int bytes) {
+    a += (unsigned)bytes;
+    asm("" : "+v"(a));
+}
 __device__ __forceinline__ float2 mkc(float x, float y) { return make_float2(x, y); }
 __device__ __forceinline__ double2 mkc(double x, double y) { return make_double2(x, y); }
 template <typename C>
@@ -856,120 +889,289 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Orders the LDS traffic of one lane group of the row FFT (SimDesc::fftShift:
-// a power of two from 8 up to the whole 256-thread block): a wavefront fence
-// for groups within one wavefront, a block barrier for a block-wide group
-// (long rows).  gs is uniform over the block.
-__device__ __forceinline__ void group_sync(int gs) {
-    if (gs > 64)
+// Orders the LDS traffic of one lane group of the row FFT: a wavefront fence
+// for groups within one wavefront, a block barrier (WIDE) for wider ones (long
+// rows).
+template <bool WIDE>
+__device__ __forceinline__ void group_sync() {
+    if constexpr (WIDE)
         __syncthreads();
     else
         wave_sync();
 }
 
-template <int RADIX, int DIR, bool HALF, typename C>
-__device__ __forceinline__ void wave_pass(const C* __restrict__ src, C* __restrict__ dst,
-                                          int M, int Ls, int lsShift, unsigned lsMagic,
-                                          const C* __restrict__ tw, int twScale, int lane,
-                                          int gs) {
-    const int nb = M / RADIX;
-    for (int b = lane; b < nb; b += gs) {
-        int k, j;
-        if (lsShift >= 0) {
-            k = b >> lsShift;
-            j = b & (Ls - 1);
-        } else {
-            k = (int)__umulhi((unsigned)b, lsMagic);  // b / Ls, exact for b < 2^16
-            j = b - k * Ls;
-        }
-        const C* in = src + j + k * Ls;
-        C x[RADIX];
+// v times the twiddle w (DIR < 0), or times its conjugate (DIR > 0).  Which
+// product each fma takes in is written out, so that a value's bits do not
+// depend on the pass that holds it.
+__device__ __forceinline__ float fmaT(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fmaT(double a, double b, double c) { return fma(a, b, c); }
+template <int DIR, typename C>
+__device__ __forceinline__ C twiddled(C v, C w) {
+    return DIR > 0 ? mkc(fmaT(v.y, w.y, v.x * w.x), fmaT(v.y, w.x, -(v.x * w.y)))
+                   : mkc(fmaT(v.x, w.x, -(v.y * w.y)), fmaT(v.y, w.x, v.x * w.y));
+}
+
+// The butterflies of one item: value q = q2 + q1 R2 goes to first-radix
+// butterfly q2.  w(t) gives the item's twiddle t, asked for in order.  The first
+// pass has j = 0 and unit twiddles in its first radix (TW1 false).
+template <int R1, int R2, int DIR, bool TW1, typename C, typename W>
+__device__ __forceinline__ void item_butterflies(C* x, const W& w) {
+    if constexpr (TW1) {
 #pragma unroll
-        for (int q = 0; q < RADIX; ++q) {
-            C v = in[q * nb];
-            if (q > 0) {
-                // a half table holds n < M only: w(n + M) = -w(n)
-                const int t = q * j * twScale;
-                C w;
-                if constexpr (HALF)
-                    w = t < M ? tw[t] : mkc(-tw[t - M].x, -tw[t - M].y);
-                else
-                    w = tw[t];
-                if (DIR > 0) w.y = -w.y;
-                v = cmul(v, w);
-            }
-            x[q] = v;
-        }
-        butterfly<RADIX, DIR>(x);
-        C* out = dst + j + k * Ls * RADIX;
+        for (int q1 = 1; q1 < R1; ++q1) {
+            const C wq = w(q1 - 1);
 #pragma unroll
-        for (int m = 0; m < RADIX; ++m) out[m * Ls] = x[m];
+            for (int q2 = 0; q2 < R2; ++q2) x[q2 + q1 * R2] = twiddled<DIR>(x[q2 + q1 * R2], wq);
+        }
+    }
+#pragma unroll
+    for (int q2 = 0; q2 < R2; ++q2) {
+        C y[R1];
+#pragma unroll
+        for (int q1 = 0; q1 < R1; ++q1) y[q1] = x[q2 + q1 * R2];
+        butterfly<R1, DIR>(y);
+#pragma unroll
+        for (int m1 = 0; m1 < R1; ++m1) x[q2 + m1 * R2] = y[m1];
+    }
+    if constexpr (R2 > 1) {
+#pragma unroll
+        for (int q2 = 1; q2 < R2; ++q2)
+#pragma unroll
+            for (int m1 = 0; m1 < R1; ++m1)
+                x[m1 * R2 + q2] = twiddled<DIR>(x[m1 * R2 + q2], w(R1 - 1 + (q2 - 1) * R1 + m1));
+#pragma unroll
+        for (int m1 = 0; m1 < R1; ++m1) {
+            C y[R2];
+#pragma unroll
+            for (int q2 = 0; q2 < R2; ++q2) y[q2] = x[m1 * R2 + q2];
+            butterfly<R2, DIR>(y);
+#pragma unroll
+            for (int m2 = 0; m2 < R2; ++m2) x[m1 * R2 + m2] = y[m2];
+        }
     }
 }
 
-// Transforms the M complex values at `row` (LDS) in place; `scratch` is the
-// calling lane group's own M-entry LDS row, `tw` the nPhi twiddles
-// exp(-2 pi i n / nPhi) staged in LDS (with HALF only the first M of them,
-// the others being w(n + M) = -w(n)), `lane` the lane within the group of gs
-// lanes.  Every lane of the wavefront (of the block, for a block-wide group)
-// calls it (rowless groups pass active = false) so that the fences and
-// barriers stay uniform.
-template <int DIR, bool HALF, typename C>
-__device__ void wave_fft(C* row, C* scratch, const C* tw, const SimDesc& s, int lane, int gs,
-                         bool active) {
-    const int M = s.M;
-    C* src = row;
-    C* dst = scratch;
-    int Ls = 1;
-    for (int p = 0; p < s.nfac; ++p) {
-        const int r = s.fac[p];
-        const int twScale = s.twStep[p];  // nPhi / (Ls r)
-        const unsigned lsMagic = s.lsMagic[p];
-        const int lsShift = ((Ls & (Ls - 1)) == 0) ? __builtin_ctz(Ls) : -1;
-        if (active) {
-            switch (r) {
-                case 2: wave_pass<2, DIR, HALF>(src, dst, M, Ls, lsShift, lsMagic, tw, twScale, lane, gs); break;
-                case 3: wave_pass<3, DIR, HALF>(src, dst, M, Ls, lsShift, lsMagic, tw, twScale, lane, gs); break;
-                case 4: wave_pass<4, DIR, HALF>(src, dst, M, Ls, lsShift, lsMagic, tw, twScale, lane, gs); break;
-                default: wave_pass<5, DIR, HALF>(src, dst, M, Ls, lsShift, lsMagic, tw, twScale, lane, gs); break;
+// Ends a pass's butterflies before the fence that follows, so that their values
+// are held across it and not their operands and twiddles (the compiler sinks
+// them to the writes otherwise: 106 VGPRs against 72, four waves per SIMD
+// against seven).
+template <int I, int R, typename C>
+__device__ __forceinline__ void pin_values(C (&x)[I][R]) {
+#pragma unroll
+    for (int it = 0; it < I; ++it)
+#pragma unroll
+        for (int q = 0; q < R; ++q) asm volatile("" : "+v"(x[it][q].x), "+v"(x[it][q].y));
+}
+
+// One pass on `row`: item b = j + k Ls (j < Ls) of nb = M / R, R = R1 R2, takes
+// the values b + q nb.  The first radix combines those M / R1 apart, twiddled
+// by w(q1 j nPhi / (Ls R1)), its outputs being Stockham positions j + m1 Ls of
+// R2 butterflies; the second combines these, twiddled by
+// w(q2 (j + m1 Ls) nPhi / (Ls R)).  The sums and products are those of two
+// separate passes.  `tw` holds the pass's twiddles in that order, j fastest,
+// so the lanes of a wavefront read them in a row.  A lane holds I items (b,
+// b + gs, ...); items past nb read item nb - 1 and write nothing.
+template <int R1, int R2, int I, int DIR, bool WIDE, typename C>
+__device__ __forceinline__ void row_pass(C* row, const C* __restrict__ tw, const FftPass& ps,
+                                         int lane, int gs, bool active) {
+    constexpr int R = R1 * R2, B = (int)sizeof(C);
+    const int nb = ps.nb, Ls = ps.Ls;
+    const unsigned rowA = lds_addr(row), twA = lds_addr(tw) + ps.tw0 * B;
+    C x[I][R];
+    int jj[I], kk[I];
+#pragma unroll
+    for (int it = 0; it < I; ++it) {
+        const int b = min(lane + it * gs, nb - 1);
+        unsigned a = rowA + b * B;
+        x[it][0] = lds_get<C>(a);
+#pragma unroll
+        for (int q = 1; q < R; ++q) {
+            lds_step(a, nb * B);
+            x[it][q] = lds_get<C>(a);
+        }
+        kk[it] = (int)(__umulhi((unsigned)b, ps.magic) + ((unsigned)b & ps.unit));
+        jj[it] = b - __mul24(kk[it], Ls);
+    }
+#pragma unroll
+    for (int it = 0; it < I; ++it) {
+        unsigned a = twA + jj[it] * B;
+        item_butterflies<R1, R2, DIR, true>(x[it], [&](int) {
+            const C w = lds_get<C>(a);
+            lds_step(a, Ls * B);
+            return w;
+        });
+    }
+    pin_values(x);
+    group_sync<WIDE>();  // every value of the row is in registers
+#pragma unroll
+    for (int it = 0; it < I; ++it) {
+        if (active && lane + it * gs < nb) {
+            unsigned a1 = rowA + (jj[it] + __mul24(kk[it], Ls * R)) * B;
+            asm volatile("" : "+v"(a1));  // the addresses are formed after the fence, not held across it
+#pragma unroll
+            for (int m2 = 0; m2 < R2; ++m2)
+#pragma unroll
+                for (int m1 = 0; m1 < R1; ++m1) {  // value m1 Ls + m2 Ls R1
+                    lds_put(a1, x[it][m1 * R2 + m2]);
+                    lds_step(a1, Ls * B);
+                }
+        }
+    }
+    group_sync<WIDE>();
+}
+
+// Transforms the M complex values at `row` (LDS) in place; `tw` holds the
+// passes' twiddles staged in LDS, `lane` is the lane within the group of gs
+// lanes.  A lane group within one wavefront needs no other wavefront; wider
+// ones (WIDE) are ordered by block barriers, so every thread of the block
+// calls this (groups without a row pass active = false).  `pv` holds the
+// passes' parameters, pass p in lane p of every wavefront.
+template <int DIR, bool WIDE, typename C>
+__device__ __forceinline__ void row_fft(C* row, const C* tw, const uint4& pv, unsigned kinds, int lane, int gs,
+                                        bool active) {
+    // a wavefront's lane groups take ascending rows
+    if (!WIDE && !__builtin_amdgcn_readfirstlane((int)active)) return;
+    int p = 0;
+    auto params = [&](int q) {
+        struct {
+            unsigned w[4];
+        } words = {{(unsigned)__builtin_amdgcn_readlane((int)pv.x, q), (unsigned)__builtin_amdgcn_readlane((int)pv.y, q),
+                    (unsigned)__builtin_amdgcn_readlane((int)pv.z, q), (unsigned)__builtin_amdgcn_readlane((int)pv.w, q)}};
+        return __builtin_bit_cast(FftPass, words);
+    };
+    FftPass ps = params(0);
+    constexpr unsigned kGroups[4] = {
+#define KAM_BIT(G, k, g) (g == G ? 1u << k : 0u) |
+#define KAM_BIT0(k, g, a, b, i) KAM_BIT(0, k, g)
+#define KAM_BIT1(k, g, a, b, i) KAM_BIT(1, k, g)
+#define KAM_BIT2(k, g, a, b, i) KAM_BIT(2, k, g)
+#define KAM_BIT3(k, g, a, b, i) KAM_BIT(3, k, g)
+        KAM_FFT_KINDS(KAM_BIT0) 0u, KAM_FFT_KINDS(KAM_BIT1) 0u, KAM_FFT_KINDS(KAM_BIT2) 0u, KAM_FFT_KINDS(KAM_BIT3) 0u};
+#define KAM_PASS(G, k, g, a, b, i)                                                  \
+    if constexpr (g == G) {                                                         \
+        if (kinds & (1u << k)) {                                                    \
+            do {                                                                    \
+                row_pass<a, b, i, DIR, WIDE>(row, tw, ps, lane, gs, active);        \
+                ps = params(++p);                                                   \
+            } while (ps.kind == k);                                                 \
+        }                                                                           \
+    }
+#define KAM_PASS0(k, g, a, b, i) KAM_PASS(0, k, g, a, b, i)
+#define KAM_PASS1(k, g, a, b, i) KAM_PASS(1, k, g, a, b, i)
+#define KAM_PASS2(k, g, a, b, i) KAM_PASS(2, k, g, a, b, i)
+#define KAM_PASS3(k, g, a, b, i) KAM_PASS(3, k, g, a, b, i)
+    if (kinds & kGroups[0]) {
+        KAM_FFT_KINDS(KAM_PASS0)
+    }
+    if (kinds & kGroups[1]) {
+        KAM_FFT_KINDS(KAM_PASS1)
+    }
+    if (kinds & kGroups[2]) {
+        KAM_FFT_KINDS(KAM_PASS2)
+    }
+    if (kinds & kGroups[3]) {
+        KAM_FFT_KINDS(KAM_PASS3)
+    }
+}
+__device__ __forceinline__ uint4 load_passes(const SimDesc& s, int tid) {
+    const Rsrc r = make_rsrc(reinterpret_cast<const float*>(s.pass), (int)sizeof(s.pass) / 4);
+    return __builtin_bit_cast(uint4, ldf4(r, 4 * (tid & 63)));
+}
+
+// The same transform for a row of M = 2^k values, with every index known but
+// the lane's (FftPow2): value i of the row sits at slot row_slot<M>(i), one
+// slot being free after every 16 (M >= 64), since the first passes write at
+// strides of 4 or 16 values, which would otherwise meet in few LDS banks.
+// With Ls, R and the item counts powers of two a slot is the sum of the slots
+// of its index's parts.
+template <int M>
+__device__ __forceinline__ constexpr int row_slot(int i) { return M >= 64 ? i + (i >> 4) : i; }
+
+template <int M, int P, int Ls, int TW0, int DIR, typename C>
+__device__ __forceinline__ void pow2_passes(C* row, const C* __restrict__ tw, int lane, bool active) {
+    typedef FftPow2<M> Plan;
+    if constexpr (P < Plan::n) {
+        constexpr int R = Plan::R[P], R2 = R / 4, NB = M / R, GS = Plan::lanes, I = (NB + GS - 1) / GS;
+        C x[I][R];
+#pragma unroll
+        for (int it = 0; it < I; ++it) {
+            const C* in = row + row_slot<M>((lane & (NB - 1)) + it * GS);
+#pragma unroll
+            for (int q = 0; q < R; ++q) x[it][q] = in[row_slot<M>(q * NB)];
+        }
+#pragma unroll
+        for (int it = 0; it < I; ++it)
+        {
+            const C* w = tw + TW0 + ((lane + it * GS) & (Ls - 1));
+            item_butterflies<4, R2, DIR, (Ls > 1)>(x[it], [&](int t) { return w[t * Ls]; });
+        }
+        pin_values(x);
+        group_sync<(GS > 64)>();
+        if (active && (NB >= GS || lane < NB)) {
+#pragma unroll
+            for (int it = 0; it < I; ++it) {
+                const int b = lane + it * GS, j = b & (Ls - 1);
+                C* out = row + row_slot<M>(j + (b - j) * R);
+#pragma unroll
+                for (int m1 = 0; m1 < 4; ++m1)
+#pragma unroll
+                    for (int m2 = 0; m2 < R2; ++m2) out[row_slot<M>(m1 * Ls + m2 * (Ls * 4))] = x[it][m1 * R2 + m2];
             }
         }
-        group_sync(gs);
-        C* tmp = src;
-        src = dst;
-        dst = tmp;
-        Ls *= r;
+        group_sync<(GS > 64)>();
+        pow2_passes<M, P + 1, Ls * R, TW0 + (R - 1) * Ls, DIR>(row, tw, lane, active);
     }
-    if (src != row) {
-        if (active)
-            for (int i = lane; i < M; i += gs) row[i] = src[i];
-        group_sync(gs);
+}
+
+template <int MC>
+__device__ __forceinline__ constexpr int fft_lanes() { return FftPow2<MC>::lanes; }
+template <>
+__device__ __forceinline__ constexpr int fft_lanes<0>() { return 1; }
+template <>
+__device__ __forceinline__ constexpr int fft_lanes<1>() { return 1; }
+
+// Row FFT of a kernel built for M = MC = 2^k values; MC = 0 and 1 take any size
+// from its plan, 1 also rows wider than a wavefront.
+template <int MC, int DIR, typename C>
+__device__ __forceinline__ void transform_row(C* row, const C* tw, const uint4& pv, unsigned kinds, int lane, int gs,
+                                              bool active) {
+    if constexpr (MC > 1) {
+        if (FftPow2<MC>::lanes > 64 || active) pow2_passes<MC, 0, 1, 0, DIR>(row, tw, lane, active);
+    } else {
+        row_fft<DIR, MC == 1>(row, tw, pv, kinds, lane, gs, active);
     }
+}
+template <int MC>
+__device__ __forceinline__ int slot_of(int i) {
+    if constexpr (MC > 1) return row_slot<MC>(i);
+    return i;
 }
 
 // Memory phases of the FFT kernels issue a batch of loads per thread before the
 // first use, so that a tile's HBM latency is paid once per batch rather than
 // once per item.
-constexpr int kDivBatch = 4;   // row points per lane in k_div_fft
+constexpr int kDivBatch = 4;   // row points per thread in k_div_fft
+constexpr int kSplitBatch = 4; // spectrum entries per thread in k_div_fft
 constexpr int kSpecBatch = 8;  // spectrum entries per thread in k_ifft_grad
 constexpr int kGradBatch = 4;  // column pairs per thread in k_ifft_grad
 
 // Workgroup size of the FFT kernels (their launches use exactly this).
 constexpr int kFftBlockShift = 8, kFftBlock = 1 << kFftBlockShift;
 
-// Stages the nPhi twiddles of s into LDS, two per float4 (nPhi is even), or
-// with `half` the first M = nPhi / 2 of them (M rounded up to even: the table
-// holds nPhi entries).
+// Stages the row FFT's pass twiddles (entries M .. 2M - 1 of the shape's table)
+// into LDS, 16 bytes at a time: two FP32 ones or one in FP64.
 __device__ __forceinline__ int tw_slots(int M) { return (M + 1) & ~1; }
-__device__ __forceinline__ void stage_twiddles(float2* twl, const SimDesc& s, int tid, int nthr,
-                                               bool half) {
-    const int n4 = (half ? tw_slots(s.M) : s.nPhi) >> 1;
-    const Rsrc tr = make_rsrc(reinterpret_cast<const float*>(s.twN), 2 * s.nPhi);
+template <typename C>
+__device__ __forceinline__ void stage_twiddles(C* twl, const SimDesc& s, int tid, int nthr) {
+    constexpr bool k64 = std::is_same<C, double2>::value;
+    const int M = s.M, n4 = k64 ? M : tw_slots(M) >> 1;
+    const Rsrc tr = k64 ? make_rsrc(reinterpret_cast<const float*>(s.twN64), 8 * M) : make_rsrc(s.twN, 4 * M);
+    const int first = k64 ? 4 * M : 2 * M;
     float4* dst = reinterpret_cast<float4*>(twl);
     for (int i0 = tid; i0 < n4; i0 += 4 * nthr) {
         float4 v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = ldf4(tr, 4 * (i0 + q * nthr));
+        for (int q = 0; q < 4; ++q) v[q] = ldf4(tr, first + 4 * (i0 + q * nthr));
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             if (i0 + q * nthr < n4) dst[i0 + q * nthr] = v[q];
@@ -984,100 +1186,120 @@ __device__ __forceinline__ void stage_twiddles(float2* twl, const SimDesc& s, in
 // four, mode-major within a block); slot 0 holds (d-hat_0, d-hat_Nyquist).
 // This is the reference's cuFFT CUFFT_INVERSE call plus shiftFKernel
 // (:640-656): d-hat_n = (1/nPhi) sum_i d_i e^{-i n i h}.
-// HALF: only the first M twiddles are staged (w(n + M) = -w(n)), and the
-// launch (k_div_fft8) asks for eight waves per SIMD; else all nPhi twiddles
-// (k_div_fft).  The two give the same values.
 // ---------------------------------------------------------------------------
-template <bool HALF>
-__device__ __forceinline__ void div_fft_tiles(const SimDesc* __restrict__ sims, const Tile* __restrict__ tiles,
-                                              int ntiles, int parity) {
+template <int MC>
+__global__ __launch_bounds__(kFftBlock) void k_div_fft(const SimDesc* __restrict__ sims,
+                                                       const Tile* __restrict__ tiles, int ntiles, int parity) {
     extern __shared__ __attribute__((aligned(16))) float2 zlds[];
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    constexpr int nthr = kFftBlock;
+    const int tid = threadIdx.x;
     for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles) {
         const Tile tile = tiles[t];
         const SimDesc& s = sims[tile.sim];
-        const int nT = s.nTheta, nP = s.nPhi, M = s.M;
+        const int nT = s.nTheta, M = MC > 1 ? MC : s.M, nP = 2 * M;
         const int j0 = tile.row0, R = tile.rows;
-        const int gsh = s.fftShift, gs = 1 << gsh;  // lanes per row (a power of two)
+        const int gsh = MC > 1 ? __builtin_ctz(fft_lanes<MC>()) : s.fftShift, gs = 1 << gsh;  // lanes per row (a power of two)
         // kFftBlock threads: kFftBlock / gs lane groups (a power of two)
         const int ngsh = kFftBlockShift - gsh, grp = tid >> gsh, ngrp = 1 << ngsh, lane = tid & (gs - 1);
-        const float* __restrict__ up = s.state[parity][F_UPHI];
-        const float* __restrict__ ut = s.state[parity][F_UTHETA];
-        const float* __restrict__ divS = s.rowf + RT_DIVS * nT;
-        const float* __restrict__ divN = s.rowf + RT_DIVN * nT;
-        const float* __restrict__ invHs = s.rowf + RT_INVHS * nT;
-        float2* twl = zlds;                                        // M or nPhi twiddles
-        float2* zbuf = zlds + (HALF ? tw_slots(M) : nP);           // R rows of M
-        float2* scratch = zbuf + (size_t)(R + grp) * M;            // this lane group's row
-        const Rsrc upR = make_rsrc(up, nT * nP), utR = make_rsrc(ut, (nT - 1) * nP);
-        const int nPass = (R + ngrp - 1) >> ngsh;                  // uniform trip count
-        for (int it = 0; it < nPass; ++it) {
-            const int r = it * ngrp + grp;
-            const bool active = r < R;
-            const int j = j0 + (active ? r : 0);
-            const float fs = divS[j], fn = divN[j], fi = invHs[j];
-            float2* row = zbuf + (size_t)(active ? r : 0) * M;
-            // kDivBatch points per lane at a time, all their loads issued
-            // before the first use; rows beyond the field (j - 1 < 0, j = nT - 1
-            // for u_theta) read as 0 through the buffer range check
-            const int on = (j - 1) * nP, oc = j * nP;
-            for (int kb = 0; kb < M; kb += kDivBatch * gs) {
-                float2 uw[kDivBatch], vn[kDivBatch], vs[kDivBatch];
-                float ue1[kDivBatch];
+        const Rsrc upR = make_rsrc(s.state[parity][F_UPHI], nT * nP);
+        const Rsrc utR = make_rsrc(s.state[parity][F_UTHETA], (nT - 1) * nP);
+        const Rsrc rowR = make_rsrc(s.rowf, RT_COUNT * nT);
+        const Rsrc specR = make_rsrc(s.spec, 2 * M * spec_rows(nT));
+        const int RS = fft_row_stride(M, MC >= 64);                // LDS row stride
+        const Rsrc twR = make_rsrc(s.twN, 4 * M);                  // w(n), n < M, at its start
+        float2* twl = zlds;                                        // the passes' twiddles
+        float2* zbuf = zlds + tw_slots(M);                         // R rows of M
+        const unsigned magicM = s.magicP2;                         // i / M, i < 2^16
+        // kDivBatch points per thread at a time, all their loads issued before
+        // the first use; rows beyond the field (j - 1 < 0, j = nT - 1 for
+        // u_theta) read as 0 through the buffer range check, points past the
+        // tile are read and not kept.  A lone wavefront pays ~5 cycles for
+        // every instruction it issues, so slots that no thread of the block
+        // needs (short tiles) are jumped over.
+        uint4 pv = make_uint4(0, 0, 0, 0);                         // the FFT passes, one per lane
+        for (int base = 0; base < R * M; base += kDivBatch * nthr) {
+            float2 uw[kDivBatch], vn[kDivBatch], vs[kDivBatch];
+            float ue1[kDivBatch], fs[kDivBatch], fn[kDivBatch], fi[kDivBatch];
+            int rq[kDivBatch], kq[kDivBatch];
 #pragma unroll
-                for (int q = 0; q < kDivBatch; ++q) {
-                    const int i0 = 2 * (kb + q * gs + lane), i2 = (i0 + 2 == nP) ? 0 : i0 + 2;
-                    uw[q] = ldf2(upR, oc + i0);
-                    ue1[q] = ldf(upR, oc + i2);
-                    vn[q] = ldf2(utR, j > 0 ? on + i0 : -1);
-                    vs[q] = ldf2(utR, oc + i0);
-                }
-                // the twiddles are staged while the first rows are in flight
-                if (it == 0 && kb == 0) stage_twiddles(twl, s, tid, nthr, HALF);
+            for (int q = 0; q < kDivBatch; ++q) {
+                if (base + q * nthr >= R * M) break;
+                const int idx = base + q * nthr + tid;
+                rq[q] = MC > 1 ? idx / M : (int)__umulhi((unsigned)idx, magicM);
+                kq[q] = idx - __mul24(rq[q], M);
+                const int j = j0 + rq[q], oc = __mul24(j, nP) , i0 = 2 * kq[q], i2 = (i0 + 2 == nP) ? 0 : i0 + 2;
+                uw[q] = ldf2(upR, oc + i0);
+                ue1[q] = ldf(upR, oc + i2);
+                vn[q] = ldf2(utR, j > 0 ? oc - nP + i0 : -1);
+                vs[q] = ldf2(utR, oc + i0);
+                fs[q] = ldf(rowR, RT_DIVS * nT + j);
+                fn[q] = ldf(rowR, RT_DIVN * nT + j);
+                fi[q] = ldf(rowR, RT_INVHS * nT + j);
+            }
+            // the twiddles are staged while the first points are in flight
+            if (base == 0 && MC <= 1) pv = load_passes(s, tid);
+            if (base == 0) stage_twiddles(twl, s, tid, nthr);
 #pragma unroll
-                for (int q = 0; q < kDivBatch; ++q) {
-                    const int k = kb + q * gs + lane;
-                    const float d0 = (fs * vs[q].x - fn * vn[q].x) + fi * (uw[q].y - uw[q].x);
-                    const float d1 = (fs * vs[q].y - fn * vn[q].y) + fi * (ue1[q] - uw[q].y);
-                    if (active && k < M) row[k] = make_float2(d0, d1);
+            for (int q = 0; q < kDivBatch; ++q) {
+                if (base + q * nthr >= R * M) break;
+                if (rq[q] < R) {
+                    const float d0 = (fs[q] * vs[q].x - fn[q] * vn[q].x) + fi[q] * (uw[q].y - uw[q].x);
+                    const float d1 = (fs[q] * vs[q].y - fn[q] * vn[q].y) + fi[q] * (ue1[q] - uw[q].y);
+                    zbuf[__mul24(rq[q], RS) + slot_of<MC>(kq[q])] = make_float2(d0, d1);
                 }
             }
-            if (it == 0) __syncthreads();  // twiddles visible to every lane group
-            group_sync(gs);
-            wave_fft<-1, HALF>(row, scratch, twl, s, lane, gs, active);
         }
-        __syncthreads();
-        float2* __restrict__ spec = reinterpret_cast<float2*>(s.spec);
-        const float2* tw = twl;
-        const float scale = 1.0f / (float)nP;
         // ceil(2^32 / R) in its 32-bit form (R = 1 splits nothing)
         const unsigned magicR = (R == 1) ? 0u : 0xffffffffu / (unsigned)R + 1u;
-        for (int idx = tid; idx < R * M; idx += nthr) {
-            const int n = (R == 1) ? idx : (int)__umulhi((unsigned)idx, magicR), r = idx - n * R, j = j0 + r;
-            const float2 Zn = zbuf[(size_t)r * M + n];
-            float2 out;
-            if (n == 0) {
-                out = make_float2((Zn.x + Zn.y) * scale, (Zn.x - Zn.y) * scale);
-            } else {
-                const float2 Zm = zbuf[(size_t)r * M + (M - n)];
-                const float2 E = make_float2(0.5f * (Zn.x + Zm.x), 0.5f * (Zn.y - Zm.y));
-                const float2 O = make_float2(0.5f * (Zn.y + Zm.y), -0.5f * (Zn.x - Zm.x));
-                const float2 X = cadd(E, cmul(tw[n], O));
-                out = cscale(X, scale);
+        auto mode = [&](int idx) { return (R == 1) ? idx : (int)__umulhi((unsigned)idx, magicR); };
+        // the first batch's split twiddles come while the rows are transformed
+        float2 wq[kSplitBatch];
+#pragma unroll
+        for (int q = 0; q < kSplitBatch; ++q) {
+            if (q * nthr >= R * M) break;
+            wq[q] = ldf2(twR, 2 * mode(tid + q * nthr));
+        }
+        __syncthreads();
+        const int nIt = (R + ngrp - 1) >> ngsh;                    // uniform trip count
+        for (int it = 0; it < nIt; ++it) {
+            const int r = it * ngrp + grp;
+            transform_row<MC, -1>(zbuf + __mul24(r < R ? r : 0, RS), twl, pv, s.passKinds, lane, gs, r < R);
+        }
+        __syncthreads();
+        const float scale = 1.0f / (float)nP;
+        for (int base = 0; base < R * M; base += kSplitBatch * nthr) {
+            if (base > 0) {
+#pragma unroll
+                for (int q = 0; q < kSplitBatch; ++q) {
+                    if (base + q * nthr >= R * M) break;
+                    wq[q] = ldf2(twR, 2 * mode(base + tid + q * nthr));
+                }
             }
-            spec[spec_index(n, j, M)] = out;
+#pragma unroll
+            for (int q = 0; q < kSplitBatch; ++q) {
+                if (base + q * nthr >= R * M) break;
+                const int idx = base + tid + q * nthr;
+                if (idx >= R * M) break;
+                const int n = mode(idx), r = idx - n * R, j = j0 + r;
+                const float2* z = zbuf + __mul24(r, RS);
+                const float2 Zn = z[slot_of<MC>(n)];
+                float2 out;
+                if (n == 0) {
+                    out = make_float2((Zn.x + Zn.y) * scale, (Zn.x - Zn.y) * scale);
+                } else {
+                    const float2 Zm = z[slot_of<MC>(M - n)];
+                    // E + w(n) O with E = (Z_n + conj Z_M-n) / 2, O = (Z_n - conj Z_M-n) / 2i
+                    const float2 O = make_float2(0.5f * (Zn.y + Zm.y), -0.5f * (Zn.x - Zm.x));
+                    const float2 X = make_float2(
+                        fmaf(0.5f, Zn.x + Zm.x, fmaf(wq[q].x, O.x, -(O.y * wq[q].y))),
+                        fmaf(0.5f, Zn.y - Zm.y, fmaf(wq[q].x, O.y, wq[q].y * O.x)));
+                    out = cscale(X, scale);
+                }
+                stf2(specR, 2 * (int)spec_index(n, j, M), out);
+            }
         }
         __syncthreads();
     }
-}
-
-__global__ __launch_bounds__(kFftBlock) void k_div_fft(const SimDesc* __restrict__ sims,
-                                                 const Tile* __restrict__ tiles, int ntiles, int parity) {
-    div_fft_tiles<false>(sims, tiles, ntiles, parity);
-}
-__global__ __launch_bounds__(kFftBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_div_fft8(
-    const SimDesc* __restrict__ sims, const Tile* __restrict__ tiles, int ntiles, int parity) {
-    div_fft_tiles<true>(sims, tiles, ntiles, parity);
 }
 
 // ---------------------------------------------------------------------------
@@ -1616,22 +1838,7 @@ __device__ __forceinline__ void load_spec(Rsrc r, int idx, double2& v) {
     v = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, idx * 16, 0, 0));
 }
 
-// Stages the first M = nPhi / 2 FP64 twiddles of s into LDS, one double2
-// (16 bytes) each; the transform takes the others as w(n + M) = -w(n).
-__device__ __forceinline__ void stage_twiddles(double2* twl, const SimDesc& s, int tid, int nthr) {
-    const Rsrc tr = make_rsrc(reinterpret_cast<const float*>(s.twN64), 4 * s.nPhi);
-    float4* dst = reinterpret_cast<float4*>(twl);
-    for (int i0 = tid; i0 < s.M; i0 += 4 * nthr) {
-        float4 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = ldf4(tr, 4 * (i0 + q * nthr));
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (i0 + q * nthr < s.M) dst[i0 + q * nthr] = v[q];
-    }
-}
-
-template <typename C, bool PONLY>
+template <typename C, bool PONLY, int MC>
 __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restrict__ sims,
                                                    const Tile* __restrict__ tiles, int ntiles,
                                                    int parity, float* __restrict__ pout) {
@@ -1639,32 +1846,32 @@ __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restri
     constexpr bool kP64 = std::is_same<C, double2>::value;
     extern __shared__ __attribute__((aligned(16))) float4 zlds4[];
     C* zlds = reinterpret_cast<C*>(zlds4);
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    constexpr int nthr = kFftBlock;
+    const int tid = threadIdx.x;
     for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles) {
         const Tile tile = tiles[t];
         const SimDesc& s = sims[tile.sim];
-        const int nT = s.nTheta, nP = s.nPhi, M = s.M;
+        const int nT = s.nTheta, M = MC > 1 ? MC : s.M, nP = 2 * M;
         const int j0 = tile.row0, R_ = tile.rows;
         const int Rp = min(R_ + 1, nT - j0);  // rows of p needed
-        const int gsh = s.fftShift, gs = 1 << gsh;  // lanes per row (a power of two)
+        const int gsh = MC > 1 ? __builtin_ctz(fft_lanes<MC>()) : s.fftShift, gs = 1 << gsh;  // lanes per row (a power of two)
         // kFftBlock threads: kFftBlock / gs lane groups (a power of two)
         const int ngsh = kFftBlockShift - gsh, grp = tid >> gsh, ngrp = 1 << ngsh, lane = tid & (gs - 1);
-        C* tw = zlds;                                               // nPhi twiddles (M in FP64)
-        C* zbuf = zlds + (kP64 ? M : nP);                           // Rp rows of M
-        C* scratch = zbuf + (size_t)(Rp + grp) * M;                 // this lane group's row
+        C* tw = zlds;                                               // the passes' twiddles
+        C* zbuf = zlds + tw_slots(M);                               // Rp rows of M
+        const int RS = fft_row_stride(M, MC >= 64);                 // LDS row stride
+        const Rsrc twR = kP64 ? make_rsrc(reinterpret_cast<const float*>(s.twN64), 8 * M) : make_rsrc(s.twN, 4 * M);
         const Rsrc specR = kP64 ? make_rsrc(s.state[parity ^ 1][0], 4 * M * nT)
                                 : make_rsrc(s.spec, 2 * M * spec_rows(nT));
-        if constexpr (kP64)
-            stage_twiddles(tw, s, tid, nthr);
-        else
-            stage_twiddles(tw, s, tid, nthr, false);
-        __syncthreads();
         // ceil(2^32 / Rp) (Rp = 1 splits nothing); idx / Rp is exact for idx < 2^16
         const unsigned magicR = (Rp == 1) ? 0u : 0xffffffffu / (unsigned)Rp + 1u;
-        for (int idx0 = tid; idx0 < Rp * M; idx0 += kSpecBatch * nthr) {
-            C Pn[kSpecBatch], Pm[kSpecBatch];
+        uint4 pv = make_uint4(0, 0, 0, 0);                          // the FFT passes, one per lane
+        for (int base = 0; base < Rp * M; base += kSpecBatch * nthr) {
+            const int idx0 = base + tid;
+            C Pn[kSpecBatch], Pm[kSpecBatch], w[kSpecBatch];
 #pragma unroll
             for (int q = 0; q < kSpecBatch; ++q) {
+                if (base + q * nthr >= Rp * M) break;  // no thread needs the slot (see k_div_fft)
                 const int idx = idx0 + q * nthr;
                 const int n = (Rp == 1) ? idx : (int)__umulhi((unsigned)idx, magicR), j = j0 + idx - n * Rp;
                 // past the spectrum (idx beyond the tile, or M - n = M) reads as 0
@@ -1677,9 +1884,14 @@ __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restri
                     load_spec(specR, (int)spec_index(n, j, M), Pn[q]);
                     load_spec(specR, (int)spec_index(M - n, j, M), Pm[q]);
                 }
+                load_spec(twR, n, w[q]);  // w(n); past M reads other entries, not used
             }
+            // the passes' twiddles are staged while the first entries are in flight
+            if (base == 0 && MC <= 1) pv = load_passes(s, tid);
+            if (base == 0) stage_twiddles(tw, s, tid, nthr);
 #pragma unroll
             for (int q = 0; q < kSpecBatch; ++q) {
+                if (base + q * nthr >= Rp * M) break;
                 const int idx = idx0 + q * nthr;
                 if (idx >= Rp * M) break;
                 const int n = (Rp == 1) ? idx : (int)__umulhi((unsigned)idx, magicR), r = idx - n * Rp;
@@ -1689,30 +1901,34 @@ __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restri
                 } else {
                     const C ev = mkc(Pn[q].x + Pm[q].x, Pn[q].y - Pm[q].y);
                     const C od = mkc(Pn[q].x - Pm[q].x, Pn[q].y + Pm[q].y);
-                    C w = tw[n];
-                    w.y = -w.y;  // exp(+i pi n / M)
-                    const C o = cmul(w, od);
+                    // exp(+i pi n / M) od, the conjugate of w(n)
+                    const C o = mkc(fmaT(w[q].x, od.x, w[q].y * od.y), fmaT(w[q].x, od.y, -(w[q].y * od.x)));
                     Y = mkc(ev.x - o.y, ev.y + o.x);
                 }
-                zbuf[(size_t)r * M + n] = Y;
+                zbuf[__mul24(r, RS) + slot_of<MC>(n)] = Y;
             }
         }
         __syncthreads();
-        const int nPass = (Rp + ngrp - 1) >> ngsh;
-        for (int it = 0; it < nPass; ++it) {
+        const int nIt = (Rp + ngrp - 1) >> ngsh;
+        for (int it = 0; it < nIt; ++it) {
             const int r = it * ngrp + grp;
-            wave_fft<+1, kP64>(zbuf + (size_t)(r < Rp ? r : 0) * M, scratch, (const C*)tw, s, lane, gs, r < Rp);
+            transform_row<MC, +1>(zbuf + __mul24(r < Rp ? r : 0, RS), (const C*)tw, pv, s.passKinds, lane, gs, r < Rp);
         }
         __syncthreads();
-        const R* p = reinterpret_cast<const R*>(zbuf);  // p[r][i], row stride nP
+        // the pair p[r][i], p[r][i + 1] (i even) sits in the slot of value i / 2, row stride PS
+        const R* p = reinterpret_cast<const R*>(zbuf);
+        const int PS = 2 * RS;
+        auto at = [&](int i) { return 2 * slot_of<MC>(i >> 1) + (i & 1); };
         if constexpr (PONLY) {
-            for (int idx = tid; idx < R_ * nP; idx += nthr) pout[(size_t)j0 * nP + idx] = (float)p[idx];
+            for (int idx = tid; idx < R_ * nP; idx += nthr) {
+                const int r = (int)__umulhi((unsigned)idx, s.magicP), i = idx - r * nP;
+                pout[(size_t)j0 * nP + idx] = (float)p[r * PS + at(i)];
+            }
             __syncthreads();
             continue;
         }
-        float* __restrict__ up = s.state[parity][F_UPHI];
-        float* __restrict__ ut = s.state[parity][F_UTHETA];
-        const Rsrc upR = make_rsrc(up, nT * nP), utR = make_rsrc(ut, (nT - 1) * nP);
+        const Rsrc upR = make_rsrc(s.state[parity][F_UPHI], nT * nP);
+        const Rsrc utR = make_rsrc(s.state[parity][F_UTHETA], (nT - 1) * nP);
         const Rsrc hsR = kP64 ? make_rsrc(reinterpret_cast<const float*>(s.rowd + RD_INVHS * nT), 2 * nT)
                               : make_rsrc(s.rowf + RT_INVHS * nT, nT);
         R invH;
@@ -1722,13 +1938,16 @@ __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restri
         // before its first store, and u_theta of the last row reads as 0
         const int half = nP >> 1, nPair = R_ * half;
         const unsigned magicH = s.magicP2;  // idx / (nPhi / 2)
-        for (int idx0 = tid; idx0 < nPair; idx0 += kGradBatch * nthr) {
+        auto row_of = [&](int idx) { return MC > 1 ? idx / M : (int)__umulhi((unsigned)idx, magicH); };
+        for (int base = 0; base < nPair; base += kGradBatch * nthr) {
+            const int idx0 = base + tid;
             float2 u[kGradBatch], v[kGradBatch];
             R hs[kGradBatch];
 #pragma unroll
             for (int q = 0; q < kGradBatch; ++q) {
+                if (base + q * nthr >= nPair) break;
                 const int idx = idx0 + q * nthr;
-                const int r = (int)__umulhi((unsigned)idx, magicH), i = 2 * (idx - r * half);
+                const int r = row_of(idx), i = 2 * (idx - r * half);
                 const int o = (j0 + r) * nP + i;
                 u[q] = ldf2(upR, o);
                 v[q] = ldf2(utR, o);
@@ -1737,21 +1956,23 @@ __global__ __launch_bounds__(kFftBlock) void k_ifft_grad(const SimDesc* __restri
             }
 #pragma unroll
             for (int q = 0; q < kGradBatch; ++q) {
+                if (base + q * nthr >= nPair) break;
                 const int idx = idx0 + q * nthr;
                 if (idx >= nPair) break;
-                const int r = (int)__umulhi((unsigned)idx, magicH), i = 2 * (idx - r * half), j = j0 + r;
+                const int r = row_of(idx), i = 2 * (idx - r * half), j = j0 + r;
                 const int il = (i == 0) ? nP - 1 : i - 1;
-                const R* pr = p + (size_t)r * nP;
-                const R p0 = pr[i], p1 = pr[i + 1];
-                const float2 nu = make_float2((float)((R)u[q].x - (p0 - pr[il]) * hs[q]),
+                const R* pr = p + __mul24(r, PS);
+                const int ia = at(i);
+                const R p0 = pr[ia], p1 = pr[ia + 1];
+                const float2 nu = make_float2((float)((R)u[q].x - (p0 - pr[at(il)]) * hs[q]),
                                               (float)((R)u[q].y - (p1 - p0) * hs[q]));
-                const size_t o = (size_t)j * nP + i;
-                *reinterpret_cast<float2*>(up + o) = nu;
+                const int o = __mul24(j, nP) + i;
+                stf2(upR, o, nu);
                 bool bad = !isfinite(nu.x) || !isfinite(nu.y);
                 if (j < nT - 1) {
-                    const float2 nv = make_float2((float)((R)v[q].x - (pr[nP + i] - p0) * invH),
-                                                  (float)((R)v[q].y - (pr[nP + i + 1] - p1) * invH));
-                    *reinterpret_cast<float2*>(ut + o) = nv;
+                    const float2 nv = make_float2((float)((R)v[q].x - (pr[PS + ia] - p0) * invH),
+                                                  (float)((R)v[q].y - (pr[PS + ia + 1] - p1) * invH));
+                    stf2(utR, o, nv);
                     bad |= !isfinite(nv.x) || !isfinite(nv.y);
                 }
                 flag_bad(s.status, bad);
@@ -1793,10 +2014,19 @@ hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, 
 }
 
 hipError_t launch_div_fft(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                          size_t ldsBytes, int gridCap, hipStream_t st, bool half) {
+                          size_t ldsBytes, int gridCap, hipStream_t st, int kernel) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(half ? k_div_fft8 : k_div_fft, dim3(grid_for(ntiles, gridCap)), dim3(kFftBlock),
-                       ldsBytes, st, sims, tiles, ntiles, parity);
+    const dim3 grid(grid_for(ntiles, gridCap)), block(kFftBlock);
+    switch (kernel) {
+#define KAM_CASE(m)                                                                                      \
+    case m:                                                                                              \
+        hipLaunchKernelGGL(k_div_fft<m>, grid, block, ldsBytes, st, sims, tiles, ntiles, parity);        \
+        break;
+        KAM_FFT_POW2(KAM_CASE)
+        KAM_CASE(1)
+#undef KAM_CASE
+        default: hipLaunchKernelGGL(k_div_fft<0>, grid, block, ldsBytes, st, sims, tiles, ntiles, parity);
+    }
     return hipGetLastError();
 }
 
@@ -1840,21 +2070,38 @@ hipError_t launch_tridiag(int lanesPerMode, int kmax, const SimDesc* sims, const
 }
 
 hipError_t launch_ifft_grad(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                            size_t ldsBytes, int gridCap, hipStream_t st, bool p64, float* pout) {
+                            size_t ldsBytes, int gridCap, hipStream_t st, int kernel, bool p64, float* pout) {
     if (ntiles <= 0) return hipSuccess;
     const dim3 grid(grid_for(ntiles, gridCap)), block(kFftBlock);
+    // the pressure readback, rare, has the kernel of any size only
     if (p64 && pout)
-        hipLaunchKernelGGL((k_ifft_grad<double2, true>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
-                           pout);
-    else if (p64)
-        hipLaunchKernelGGL((k_ifft_grad<double2, false>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
+        hipLaunchKernelGGL((k_ifft_grad<double2, true, 1>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
                            pout);
     else if (pout)
-        hipLaunchKernelGGL((k_ifft_grad<float2, true>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
+        hipLaunchKernelGGL((k_ifft_grad<float2, true, 1>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
                            pout);
     else
-        hipLaunchKernelGGL((k_ifft_grad<float2, false>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity,
-                           pout);
+        switch (p64 ? -kernel : kernel) {
+#define KAM_CASE(m)                                                                                            \
+    case m:                                                                                                    \
+        hipLaunchKernelGGL((k_ifft_grad<float2, false, m>), grid, block, ldsBytes, st, sims, tiles, ntiles,    \
+                           parity, pout);                                                                      \
+        break;                                                                                                 \
+    case -m:                                                                                                   \
+        hipLaunchKernelGGL((k_ifft_grad<double2, false, m>), grid, block, ldsBytes, st, sims, tiles, ntiles,   \
+                           parity, pout);                                                                      \
+        break;
+            KAM_FFT_POW2(KAM_CASE)
+            KAM_CASE(1)
+#undef KAM_CASE
+            default:
+                if (p64)
+                    hipLaunchKernelGGL((k_ifft_grad<double2, false, 0>), grid, block, ldsBytes, st, sims, tiles,
+                                       ntiles, parity, pout);
+                else
+                    hipLaunchKernelGGL((k_ifft_grad<float2, false, 0>), grid, block, ldsBytes, st, sims, tiles,
+                                       ntiles, parity, pout);
+        }
     return hipGetLastError();
 }
 
@@ -1872,10 +2119,13 @@ static hipError_t allow_lds(const void* fn, size_t bytes) {
 }
 
 hipError_t configure_kernels(size_t bytes) {
-    const void* fns[] = {(const void*)k_advect<adv_stride(64)>, (const void*)k_advect<adv_stride(128)>,
-                         (const void*)k_div_fft, (const void*)k_ifft_grad<float2, false>,
-                         (const void*)k_ifft_grad<double2, false>, (const void*)k_ifft_grad<float2, true>,
-                         (const void*)k_ifft_grad<double2, true>};
+#define KAM_FNS(m)                                                                     \
+    (const void*)k_div_fft<m>, (const void*)k_ifft_grad<float2, false, m>,             \
+        (const void*)k_ifft_grad<double2, false, m>,
+    const void* fns[] = {KAM_FFT_POW2(KAM_FNS) KAM_FNS(0) KAM_FNS(1)(const void*) k_advect<adv_stride(64)>,
+                         (const void*)k_advect<adv_stride(128)>, (const void*)k_ifft_grad<float2, true, 1>,
+                         (const void*)k_ifft_grad<double2, true, 1>};
+#undef KAM_FNS
     for (const void* fn : fns) {
         const hipError_t e = allow_lds(fn, bytes);
         if (e != hipSuccess) return e;

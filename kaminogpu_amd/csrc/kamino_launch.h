@@ -13,12 +13,20 @@ namespace kam {
 constexpr int kAdvHaloRows = 3, kAdvHaloCols = 4, kAdvMaxCols = 128, kAdvMaxRows = 64;
 constexpr int adv_stride(int W) { return (W <= 64 ? 64 : 128) + 2 * kAdvHaloCols; }
 
+// LDS row stride, in complex values, of a row of M in the row FFT.  Four past
+// its end, so that the rows of a tile start in different banks (the spectrum
+// is read and written across them); with `padded` (the kernels of one
+// power-of-two size) one slot is left free after every 16 values too.
+constexpr int fft_row_stride(int M, bool padded) { return M + (padded ? M >> 4 : 0) + 4; }
+
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                          int stride, size_t ldsBytes, int gridCap, hipStream_t st);
 hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                             int gridCap, hipStream_t st);
+// kernel: M where every row FFT of the launch has the same length M = 2^k >= 32
+// (FftPow2); else 1 when some rows span wavefronts, 0 when none does.
 hipError_t launch_div_fft(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                          size_t ldsBytes, int gridCap, hipStream_t st, bool half);
+                          size_t ldsBytes, int gridCap, hipStream_t st, int kernel);
 // `parity` names the current state copy: a simulation with the FP64 pressure
 // keeps its solved spectrum over the other one.
 // fp32: run the elimination in FP32 with subtraction-free pivots (the FP32
@@ -30,7 +38,7 @@ hipError_t launch_tridiag(int lanesPerMode, int kmax, const SimDesc* sims, const
 // pout (one simulation only): write its pressure rows there instead of
 // updating the velocities.
 hipError_t launch_ifft_grad(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                            size_t ldsBytes, int gridCap, hipStream_t st, bool p64 = false,
+                            size_t ldsBytes, int gridCap, hipStream_t st, int kernel, bool p64 = false,
                             float* pout = nullptr);
 
 // The phi transforms of SIM_DFT simulations (kamino_dft.hip): divergence rows

@@ -23,11 +23,16 @@ int set_err(int code, const char* fmt, ...);
             return ::kam::set_err(KAM_EHIP, "%s: %s", #call, hipGetErrorString(e_)); \
     } while (0)
 
+// Passes and lanes per row of the row FFT of M complex values.
+struct FftPlan {
+    int nPass = 0, lanes = 0;
+    FftPass pass[kFftMaxPass + 1] = {};
+};
+
 // Launch geometry of one simulation shape.
 struct Plan {
     int nT = 0, nP = 0, M = 0;
-    int nfac = 0;
-    int fac[12] = {0};
+    FftPlan fft;
     int advRows = 0;   // rows per advection tile
     int advCols = 0;   // columns per advection tile
     int fftRows = 0;   // rows per FFT tile
@@ -65,7 +70,8 @@ int acquire_tables(int device, int nTheta, double dt, double radius, Tables* out
 void release_tables(int device, int nTheta, double dt, double radius);
 
 // Host values of the per-shape tables (no allocation): rowf[RT_COUNT * nT],
-// rowd[RD_COUNT * nT], tw[2 nPhi] (FP32) and tw64[2 nPhi] (FP64).
+// rowd[RD_COUNT * nT], and the twiddles (SimDesc::twN) tw[2 nPhi] (FP32) and
+// tw64[2 nPhi] (FP64).
 void compute_tables(int nTheta, double dt, double radius, float* rowf, double* rowd, float* tw,
                     double* tw64);
 
@@ -93,7 +99,7 @@ struct TileLayout {
     int ntri = 0;
     TriClass tri[12] = {};
     size_t advLds = 0, fftLds = 0, fftLds64 = 0, divLds = 0;
-    bool divW8 = false;  // forward transform by k_div_fft8 (half twiddle table, eight waves)
+    int fftKernel = 0;  // the transform kernels' variant (launch_div_fft)
     int advStride = 0;  // staged row stride of the advection launch
 };
 

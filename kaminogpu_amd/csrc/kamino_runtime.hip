@@ -63,30 +63,114 @@ static size_t adv_lds(int R, int W, int SW, bool geometric) {
     const size_t uv = geometric ? (size_t)(R + 1) * (W + 2) + (R + 2) * (W + 1) + 2 * (W + 1) : 0;
     return (2 * plane + std::max(plane, uv) + 3 * (size_t)(R + 2) + 3 * (256 / 64)) * sizeof(float);
 }
-// Lanes per row in the row FFT (a quarter of M, 8..64, power of two); a
-// 256-thread block holds 256 / group lane groups, each with a scratch row.
-// Long rows (M >= 1024) take the whole block per row, its passes ordered by
-// block barriers: a 1024 x 2048 sphere has only four rows per CU, so with
-// one wavefront per row each SIMD would hold a single transform's chain.
-static int fft_group_host(int M) {
-    if (M >= 1024) return 256;
-    int g = 8;
-    while (g < 64 && 4 * g < M) g *= 2;
-    return g;
+// The elementary radices and items per lane of each kind of FFT pass.
+struct Radices {
+    int R1, R2, I;
+};
+#define KAM_KIND(k, g, a, b, i) {a, b, i},
+static constexpr Radices kRadices[] = {{1, 1, 0}, KAM_FFT_KINDS(KAM_KIND)};  // by kind
+#undef KAM_KIND
+static constexpr int kRadixKinds = (int)(sizeof(kRadices) / sizeof(kRadices[0]));
+
+// Cycles a wavefront issues for one item of a pass (butterflies, twiddles and
+// their LDS reads, addresses), roughly: what the plan search below weighs.
+static int pass_issue(int R1, int R2) {
+    auto bfly = [](int r) { return r == 2 ? 4 : (r == 5 ? 40 : 16); };
+    const int tw = (R1 - 1) * R2 + (R2 - 1) * R1, rd = (R1 - 1) + (R2 - 1) * R1;
+    return 4 * (R2 * bfly(R1) + (R2 > 1 ? R1 * bfly(R2) : 0) + 5 * tw + 3 * rd + 2 * R1 * R2 + 12);
 }
-// LDS of an inverse-transform tile: the nPhi = 2M twiddles (M in FP64), R + 1
-// rows of M complex and the lane groups' scratch rows; FP32 complex (8 bytes),
-// or FP64 (16 bytes) for the FP64 pressure
+
+// The row FFT's passes and lanes per row.  The elementary radices of M stay in
+// their order (factor_m), so the sums and products of a transform, and with
+// them its bits, do not depend on the plan; neighbours may share a pass
+// (KAM_FFT_KINDS), which saves an LDS round trip, and a row may take 8 to 256
+// lanes.  Many lanes shorten one row's chain (a launch of one sphere has few
+// rows), few let a wavefront hold several rows.  The plan minimises the
+// estimated cycles of a row plus half of those times the share of a wavefront
+// that it takes; a pass costs its issue and about 350 cycles of LDS round trip
+// and control, 150 more where a row spans wavefronts and block barriers order
+// it.  (Weights 0 to 2 in place of the half time within 3% of each other.)
+static void add_pass(FftPlan& pl, int M, int kind, int& Ls, int& tw0) {
+    const int R = kRadices[kind].R1 * kRadices[kind].R2;
+    FftPass& ps = pl.pass[pl.nPass++];
+    ps.kind = (uint16_t)kind;
+    ps.nb = (uint16_t)(M / R);
+    ps.Ls = (uint16_t)Ls;
+    ps.tw0 = (uint16_t)tw0;
+    ps.magic = Ls == 1 ? 0u : (unsigned)((((uint64_t)1 << 32) + Ls - 1) / Ls);
+    ps.unit = Ls == 1 ? ~0u : 0u;
+    tw0 += (R - 1) * Ls;
+    Ls *= R;
+}
+// The kind with the fewest items per lane that hold `items` (-1: none).
+static int pass_kind(int R1, int R2, int items) {
+    int best = -1;
+    for (int q = 1; q < kRadixKinds; ++q)
+        if (kRadices[q].R1 == R1 && kRadices[q].R2 == R2 && kRadices[q].I >= items &&
+            (best < 0 || kRadices[q].I < kRadices[best].I))
+            best = q;
+    return best;
+}
+template <int M>
+static void plan_pow2(FftPlan& pl) {
+    typedef FftPow2<M> P;
+    pl = FftPlan();
+    pl.lanes = P::lanes;
+    int Ls = 1, tw0 = 0;
+    for (int p = 0; p < P::n; ++p) {
+        const int R = P::R[p];
+        add_pass(pl, M, pass_kind(4, R / 4, (M / R + P::lanes - 1) / P::lanes), Ls, tw0);
+    }
+}
+static void plan_fft(int M, const int* fac, int nfac, FftPlan& best) {
+    switch (M) {
+#define KAM_CASE(m) \
+    case m: plan_pow2<m>(best); return;
+        KAM_FFT_POW2(KAM_CASE)
+#undef KAM_CASE
+    }
+    double bestCost = 1e300;
+    for (int lanes = 8; lanes <= 256; lanes *= 2) {
+        // bit k of cut: a pass boundary after factor k
+        for (int cut = 0; cut < (1 << (nfac - 1)); ++cut) {
+            FftPlan pl;
+            pl.lanes = lanes;
+            int Ls = 1, tw0 = 0;
+            double lat = 0;
+            bool ok = true;
+            for (int f = 0; ok && f < nfac;) {
+                const int R1 = fac[f];
+                const bool two = f + 1 < nfac && !((cut >> f) & 1);
+                if (two && f + 2 < nfac && !((cut >> (f + 1)) & 1)) ok = false;  // at most two to a pass
+                const int R2 = two ? fac[f + 1] : 1, items = (M / (R1 * R2) + lanes - 1) / lanes;
+                const int kind = pass_kind(R1, R2, items);
+                // kinds in rising order (KAM_FFT_KINDS)
+                if (!ok || kind < 0 || pl.nPass == kFftMaxPass || (pl.nPass > 0 && kind < pl.pass[pl.nPass - 1].kind)) {
+                    ok = false;
+                    break;
+                }
+                add_pass(pl, M, kind, Ls, tw0);
+                lat += items * pass_issue(R1, R2) + 350 + (lanes > 64 ? 150 : 0);
+                f += two ? 2 : 1;
+            }
+            const double cost = lat * (1.0 + 0.5 * lanes / 64.0);
+            if (ok && cost < bestCost) {
+                bestCost = cost;
+                best = pl;
+            }
+        }
+    }
+}
+// LDS row stride of a transform row in complex values
+static int fft_stride(int M) { return fft_row_stride(M, (M & (M - 1)) == 0 && M >= 64); }
+// LDS of an inverse-transform tile: the passes' twiddles and R + 1 rows; FP32
+// complex (8 bytes), or FP64 (16 bytes) for the FP64 pressure
 static size_t fft_lds(int R, int M, bool p64 = false) {
-    return (size_t)((p64 ? 1 : 2) + R + 1 + 256 / fft_group_host(M)) * M * (p64 ? 16 : 8);
+    return ((size_t)((M + 1) & ~1) + (size_t)(R + 1) * fft_stride(M)) * (p64 ? 16 : 8);
 }
-// LDS of a forward-transform tile: the nPhi = 2M twiddles (k_div_fft) or the
-// first M of them rounded up to even (k_div_fft8, `half`), R rows of M complex
-// and the scratch rows; with half twiddles 18 KiB at 4 x 256, eight
-// workgroups per CU
-static size_t div_lds(int R, int M, bool half) {
-    const size_t tw = half ? (size_t)((M + 1) & ~1) : (size_t)2 * M;
-    return (tw + (size_t)(R + 256 / fft_group_host(M)) * M) * 8;
+// LDS of a forward-transform tile: the passes' twiddles and R rows
+static size_t div_lds(int R, int M) {
+    return ((size_t)((M + 1) & ~1) + (size_t)R * fft_stride(M)) * 8;
 }
 static constexpr size_t kLdsMax = 160 * 1024;
 
@@ -130,8 +214,9 @@ int make_plan(int nT, int nP, Plan& p) {
     p.nT = nT;
     p.nP = nP;
     p.M = nP / 2;
-    p.nfac = factor_m(p.M, p.fac);
-    if (p.nfac < 0)
+    int fac[12] = {0};
+    const int nfac = factor_m(p.M, fac);
+    if (nfac < 0)
         return set_err(KAM_EINVAL, "n_theta must factor as 2^a 3^b 5^c (got %d)", nT);
     // advection tile: 16 rows x 64 columns (8 rows below nTheta = 128), about
     // 22 KiB of LDS, the shape the autotuner picks for most sizes of a mixed
@@ -140,14 +225,13 @@ int make_plan(int nT, int nP, Plan& p) {
     // mixed batches compact.
     p.advCols = nP < 64 ? nP : 64;
     p.advRows = nT < 128 ? (nT < 8 ? nT : 8) : 16;
-    // FFT tile: at most 8 rows (+1 halo row for the inverse, + scratch rows) in ~48 KiB
-    int Rf = (int)(49152 / (8 * (size_t)p.M)) - 3 - 256 / fft_group_host(p.M);
-    Rf = Rf < 1 ? 1 : (Rf > 8 ? 8 : Rf);
-    // long rows (a block per row): one row per tile.  The inverse transform
-    // then repeats its halo row, but twice as many tiles run at once
-    // (measured, ms per step at one sphere: 1024 x 2048 0.0811 with two rows
-    // -> 0.0798, 2048 x 4096 0.314 -> 0.272)
-    if (fft_group_host(p.M) == 256) Rf = 1;
+    plan_fft(p.M, fac, nfac, p.fft);
+    // FFT tile (the inverse adds a halo row): about four points per thread of
+    // the forward transform.  Measured, us per step (FFT rows): 128 spheres of
+    // 256 x 512 300 (2), 294 (4), 299 (8); 256 of 128 x 256 154 (4), 152 (8);
+    // 32 of 405 x 810 220 (2), 216 (4); 32 of 512 x 1024 306 (2), 303 (4); 8 of
+    // 1024 x 2048 310 (1), 304 (2), 310 (3); 2 of 2048 x 4096 356 (1), 359 (2)
+    const int Rf = p.M <= 192 ? 8 : (p.M <= 640 ? 4 : (p.M <= 1280 ? 2 : 1));
     p.fftRows = Rf > nT ? nT : Rf;
     // tridiagonal: L lanes per mode, at most K rows per lane
     if (nT <= 64) { p.triL = 8; p.triK = 8; }
@@ -235,22 +319,31 @@ void compute_tables(int nT, double dt, double radius, float* rowf, double* rowd,
         rowf[RT_TRIC * nT + j] = (j == nT - 1) ? 0.f : (float)(h2 + ct);
         rowf[RT_TRIS * nT + j] = (float)rowd[RD_INVSIN2 * nT + j];
     }
-    // exp(-2 pi i n / nPhi); the second half is the exact negation of the
-    // first (w(n + M) = -w(n)), so kernels that stage only the first half
-    // read the same values as those that stage all of it
+    // w(n) = exp(-2 pi i n / nPhi) for n < M; w(n + M) = -w(n) exactly
     const int M = nP / 2;
-    for (int n = 0; n < nP; ++n) {
-        if (n < M) {
-            const double a = 2.0 * kPi * n / nP;
-            tw64[2 * n] = std::cos(a);
-            tw64[2 * n + 1] = -std::sin(a);
-        } else {
-            tw64[2 * n] = -tw64[2 * (n - M)];
-            tw64[2 * n + 1] = -tw64[2 * (n - M) + 1];
-        }
-        tw[2 * n] = (float)tw64[2 * n];
-        tw[2 * n + 1] = (float)tw64[2 * n + 1];
+    auto w = [&](int n, double* out) {
+        const double a = 2.0 * kPi * (n < M ? n : n - M) / nP, sign = n < M ? 1.0 : -1.0;
+        out[0] = sign * std::cos(a);
+        out[1] = -sign * std::sin(a);
+    };
+    for (int n = 0; n < M; ++n) w(n, tw64 + 2 * n);
+    // then the passes' twiddles: of each pass those of its first radix, then
+    // of its second (row_pass), for j = 0 .. Ls - 1 in a row
+    FftPlan pl;
+    int fac[12] = {0};
+    plan_fft(M, fac, factor_m(M, fac), pl);
+    double* t = tw64 + 2 * M;
+    for (int p = 0; p < pl.nPass; ++p) {
+        const Radices r = kRadices[pl.pass[p].kind];
+        const int Ls = pl.pass[p].Ls;
+        for (int q = 1; q < r.R1; ++q)
+            for (int j = 0; j < Ls; ++j, t += 2) w(q * j * (nP / (Ls * r.R1)), t);
+        for (int q = 1; q < r.R2; ++q)
+            for (int j = 0; j < r.R1 * Ls; ++j, t += 2) w(q * j * (nP / (Ls * r.R1 * r.R2)), t);
     }
+    t[0] = 1.0;  // M - 1 of them: one entry is free
+    t[1] = 0.0;
+    for (int n = 0; n < 2 * nP; ++n) tw[n] = (float)tw64[n];
 }
 
 int acquire_tables(int device, int nT, double dt, double radius, Tables* out) {
@@ -425,15 +518,10 @@ void fill_desc(SimDesc& d, const Plan& p, const Tables& t, const kam_sim_desc& s
     d.rowd = t.rowd;
     d.twN = t.twN;
     d.twN64 = t.twN64;
-    d.nfac = p.nfac;
-    int Ls = 1;
-    for (int k = 0; k < p.nfac; ++k) {
-        d.fac[k] = p.fac[k];
-        d.twStep[k] = p.nP / (Ls * p.fac[k]);
-        d.lsMagic[k] = (Ls & (Ls - 1)) == 0 ? 0u : (unsigned)((((uint64_t)1 << 32) + Ls - 1) / Ls);
-        Ls *= p.fac[k];
-    }
-    d.fftShift = __builtin_ctz((unsigned)fft_group_host(p.M));
+    std::memcpy(d.pass, p.fft.pass, sizeof d.pass);
+    d.passKinds = 0;
+    for (int k = 0; k < p.fft.nPass; ++k) d.passKinds |= 1u << p.fft.pass[k].kind;
+    d.fftShift = __builtin_ctz((unsigned)p.fft.lanes);
     d.advRows = p.advRows;
     d.fftRows = p.fftRows;
     d.magicP = (unsigned)((((uint64_t)1 << 32) + (uint64_t)p.nP - 1) / (uint64_t)p.nP);
@@ -578,9 +666,8 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     // FP64 pressure, whose inverse transform is a launch of its own (FP64 rows
     // in LDS: their tiles hold as many rows as fit)
     L.fftOff = cnt;
-    // the eight-wave forward kernel when every FFT simulation asks for it
-    bool anyFft = false, allW8 = true;
-    size_t divFull = 0, divHalf = 0;
+    int commonM = -1;   // M of every simulation (0: several)
+    bool wideRows = false;  // rows of more than one wavefront
     for (int pass = 0; pass < 2; ++pass)
         for (int s = 0; s < n; ++s) {
             const Plan& p = plans[s];
@@ -594,14 +681,12 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
                 L.nFft64 += p64 ? 1 : 0;
             }
             L.fftLds = std::max(L.fftLds, fft_lds(R, p.M));
-            divFull = std::max(divFull, div_lds(R, p.M, false));
-            divHalf = std::max(divHalf, div_lds(R, p.M, true));
-            anyFft = true;
-            allW8 = allW8 && p.transform == KAM_TRANSFORM_FFT8;
+            L.divLds = std::max(L.divLds, div_lds(R, p.M));
+            commonM = (commonM < 0 || commonM == p.M) ? p.M : 0;
+            wideRows = wideRows || p.fft.lanes > 64;
             if (p64) L.fftLds64 = std::max(L.fftLds64, fft_lds(R, p.M, true));
         }
-    L.divW8 = anyFft && allW8;
-    L.divLds = L.divW8 ? divHalf : divFull;
+    L.fftKernel = (commonM >= 32 && (commonM & (commonM - 1)) == 0) ? commonM : (wideRows ? 1 : 0);
     L.nFft = cnt - L.fftOff;
     L.nFft32 = L.nFft - L.nFft64;
     // SIM_DFT simulations: row runs for the divergence and gradient kernels,
@@ -695,7 +780,7 @@ int launch_step(const SimDesc* dSims, const Tile* dTiles, const TileLayout& L, i
     }
     if (phases & KAM_PHASE_DIVFFT) {
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_DIVFFT], st));
-        KAM_HIP(launch_div_fft(dSims, dTiles + L.fftOff, L.nFft, p, L.divLds, kGridCap, st, L.divW8));
+        KAM_HIP(launch_div_fft(dSims, dTiles + L.fftOff, L.nFft, p, L.divLds, kGridCap, st, L.fftKernel));
         KAM_HIP(launch_dft_forward(dSims, dTiles + L.dftRowOff, L.nDftRow, dTiles + L.dftOff, L.nDft, p, st));
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_DIVFFT + 1], st));
     }
@@ -707,9 +792,9 @@ int launch_step(const SimDesc* dSims, const Tile* dTiles, const TileLayout& L, i
     }
     if (phases & KAM_PHASE_IFFT) {
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_IFFT], st));
-        KAM_HIP(launch_ifft_grad(dSims, dTiles + L.fftOff, L.nFft32, p, L.fftLds, kGridCap, st, false));
+        KAM_HIP(launch_ifft_grad(dSims, dTiles + L.fftOff, L.nFft32, p, L.fftLds, kGridCap, st, L.fftKernel, false));
         KAM_HIP(launch_ifft_grad(dSims, dTiles + L.fftOff + L.nFft32, L.nFft64, p, L.fftLds64, kGridCap, st,
-                                 true));
+                                 L.fftKernel, true));
         KAM_HIP(launch_dft_inverse(dSims, dTiles + L.dftRowOff, L.nDftRow, dTiles + L.dftOff, L.nDft, p, st));
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_IFFT + 1], st));
     }
@@ -749,9 +834,9 @@ int DeviceBatch::launch_tri_residual(hipStream_t st, int parity) {
 
 int DeviceBatch::launch_pressure(hipStream_t st, int parity, float* pout) {
     const TileLayout& L = lay_;
-    KAM_HIP(launch_ifft_grad(dSims_, dTiles_ + L.fftOff, L.nFft32, parity, L.fftLds, kGridCap, st, false, pout));
+    KAM_HIP(launch_ifft_grad(dSims_, dTiles_ + L.fftOff, L.nFft32, parity, L.fftLds, kGridCap, st, L.fftKernel, false, pout));
     KAM_HIP(launch_ifft_grad(dSims_, dTiles_ + L.fftOff + L.nFft32, L.nFft64, parity, L.fftLds64, kGridCap, st,
-                             true, pout));
+                             L.fftKernel, true, pout));
     KAM_HIP(launch_dft_pressure(dSims_, dTiles_ + L.dftOff, L.nDft, parity, st));
     return KAM_OK;
 }
