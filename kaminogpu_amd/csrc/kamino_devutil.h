@@ -25,6 +25,18 @@ __device__ __forceinline__ double ldd(Rsrc r, int elem) {
 __device__ __forceinline__ float4 ldf4(Rsrc r, int elem) {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, elem * 4, 0, 0));
 }
+// BYTES (4 or 16) per lane from element `elem` on, straight into LDS: lane l of
+// the wavefront writes at dst + l BYTES (dst is the same in all its lanes).
+// Counts as a vector memory load; wait for it before a barrier.
+template <int BYTES>
+__device__ __forceinline__ void load_to_lds(Rsrc r, float* dst, int elem) {
+    static_assert(BYTES == 4 || BYTES == 16, "dword or dwordx4");
+    __attribute__((address_space(3))) void* d = (__attribute__((address_space(3))) void*)dst;
+    if constexpr (BYTES == 16)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, d, 16, elem * 4, 0, 0, 0);
+    else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, d, 4, elem * 4, 0, 0, 0);
+}
 // A store at byte offset vbytes + sbytes: a row walk passes the lane's column
 // in vbytes (loop-invariant) and the row's base in sbytes (a scalar), so the
 // address costs no vector instruction.  Stores past the range are dropped.

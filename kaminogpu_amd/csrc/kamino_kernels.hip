@@ -351,11 +351,80 @@ __device__ __forceinline__ float advect_node_fast(const float* __restrict__ S, i
     return sample_fast<SW>(bs, fmaf(-(u0p + ump), hP, sP), fmaf(-(u0t + umt), hT, sT));
 }
 
-// Unsigned maximum over the 64 lanes of a wavefront.
+// ---------------------------------------------------------------------------
+// Tiles whose stencils reach a pole (within kER rows of it) stage a wider
+// window: columns [c0 - D, c0 + W + D) and, beside it, the same columns half a
+// turn away.  A stencil folded over the pole, or a pole row's second row, then
+// sits at a fixed distance from the unfolded one, so the pole rules cost
+// selects on an LDS offset, and every lane of a wavefront takes the same path.
+// (With samples that fall back to global gathers, a polar tile ran three paths
+// per sample one after another and took 22000 to 28000 cycles against 10000 to
+// 12000 of the others, which was the launch's time on one sphere.)  Values
+// outside the window (faster flows than D holds) come from the global sampler;
+// both read the same values with the same weights.
+// ---------------------------------------------------------------------------
+struct PolarStage {
+    const float* S;         // staged field k at S + k * plane
+    int plane, stride;      // stride = 2 win
+    int win;                // columns of the window; the antipodal one follows it
+    int rlo, rows[3];       // first staged row; staged rows of each Kind
+};
+
+// lc: the node's column in its window; blk: the window (1: antipodal).
+template <int KIND>
+__device__ __forceinline__ float sample_polar(const PolarStage& ps, Rsrc f, const Grid& g, int bi, int lc, int blk,
+                                              float fphi, int bj, float fth) {
+    const int poleRow = (KIND == K_VTHETA) ? g.nT - 2 : g.nT - 1;
+    const int lp = lc + cell_of(fphi), j = bj + cell_of(fth);
+    const float ap = frac_of(fphi), fr = frac_of(fth);
+    const int part = fr > 0.f ? 1 : 0;
+    // fold: t < 0 -> -t and t > nTheta -> 2 nTheta - t, each half a turn away
+    const bool neg = j < 0, flip = neg | (j + part > g.nT);
+    const int jt = flip ? (neg ? 0 : 2 * g.nT) - j - part : j;
+    const float at = (flip && part) ? 1.f - fr : fr;
+    const bool pole = ((jt == 0) & flip) | (jt == poleRow);
+    const int jr = jt - ps.rlo;
+    // both rows staged (the pole branch reads one row twice), both columns too
+    const bool inside = ((unsigned)jr < (unsigned)(ps.rows[KIND] - (pole ? 0 : 1))) &
+                        ((unsigned)lp < (unsigned)(ps.win - 1));
+    if (!inside) return sample<KIND>(f, g, bi, fphi, bj, fth);
+    const int here = ((flip ? 1 : 0) ^ blk) ? ps.win : 0;
+    const float* q = ps.S + KIND * ps.plane + __mul24(jr, ps.stride) + lp + here;
+    const float* r = q + (pole ? ps.win - 2 * here : ps.stride);
+    const float w = pole ? ((KIND == K_VPHI) ? at : 0.5f * at) : at;
+    return lerpf(lerpf(q[0], q[1], ap), lerpf(r[0], r[1], ap), w);
+}
+
+// advect_node in a polar window: node (i, j), at column lc of window blk.
+template <int NODE>
+__device__ __forceinline__ float advect_node_polar(const PolarStage& ps, Rsrc up, Rsrc ut, Rsrc src, const Grid& g,
+                                                   int i, int j, int lc, int blk, float hP, float hT) {
+    static_assert(kNodeP[NODE] + kShiftP[NODE] == 0.f && kNodeT[NODE] + kShiftT[NODE] == 0.f, "own lattice");
+    constexpr float pP = kNodeP[NODE] + kShiftP[K_VPHI], pT = kNodeT[NODE] + kShiftT[K_VPHI];
+    constexpr float tP = kNodeP[NODE] + kShiftP[K_VTHETA], tT = kNodeT[NODE] + kShiftT[K_VTHETA];
+    const float* node = ps.S + __mul24(j - ps.rlo, ps.stride) + lc + (blk ? ps.win : 0);
+    const float u0p = (NODE == K_VPHI) ? node[0] : sample_polar<K_VPHI>(ps, up, g, i, lc, blk, pP, j, pT);
+    const float u0t = (NODE == K_VTHETA) ? node[ps.plane] : sample_polar<K_VTHETA>(ps, ut, g, i, lc, blk, tP, j, tT);
+    const float ump = sample_polar<K_VPHI>(ps, up, g, i, lc, blk, fmaf(-u0p, hP, pP), j, fmaf(-u0t, hT, pT));
+    const float umt = sample_polar<K_VTHETA>(ps, ut, g, i, lc, blk, fmaf(-u0p, hP, tP), j, fmaf(-u0t, hT, tT));
+    // a field sampled at a departure from its own node
+    return sample_polar<NODE>(ps, src, g, i, lc, blk, fmaf(-(u0p + ump), hP, 0.f), j, fmaf(-(u0t + umt), hT, 0.f));
+}
+
+// Unsigned maximum over the 64 lanes of a wavefront, in lane 63: within rows of
+// 16 lanes, then across them, by DPP moves (shuffles through LDS took 6 x 60
+// cycles each).  Lanes without a source keep their own value.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned dpp_max(unsigned v) {
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false));
+}
 __device__ __forceinline__ unsigned wave_max(unsigned v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, m, 64));
-    return v;
+    v = dpp_max<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_max<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_max<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_max<0x118, 0xf>(v);  // row_shr:8
+    v = dpp_max<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_max<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 constexpr int kAdvWaves = 256 / 64;  // wavefronts of an advection workgroup
 
@@ -383,7 +452,7 @@ constexpr float kFastDPhi = 2.4f, kFastDTheta = 1.4f;
 template <int SW>
 __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims,
                                                 const Tile* __restrict__ tiles, int ntiles,
-                                                int parity) {
+                                                int parity, int polarD) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int nthr = kAdvWaves * 64;  // launch_advect's block size
     const int tid = threadIdx.x;
@@ -415,8 +484,12 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         };
 
         // ---- stage rows j0-kER .. j0+R+kER-1, columns c0-kEC .. c0+W+kEC-1
-        const int SR = R + 2 * kER, SC = W + 2 * kEC, plane = SR * SW;
-        const int js = j0 - kER;
+        // (a polar tile: only rows of the sphere, and its two windows, see PolarStage)
+        const bool geom = (s.flags & SIM_GEOMETRIC) != 0;
+        const bool polar = j0 < kER + 1 || j0 + R > nT - kER - 1;
+        const int js = j0 - kER, SR = R + 2 * kER, SC = W + 2 * kEC;
+        const int rlo = max(0, js), win = W + 2 * polarD;
+        const int plane = polar ? (min(nT, js + SR) - rlo) * 2 * win : SR * SW;
         Stage st;
         st.S = lds;
         st.plane = plane;
@@ -433,9 +506,9 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         // u_theta nodes) and the geometric coefficient G of those rows, after
         // the staged planes and the advected u block
         const int W1 = W + 1, W2 = W + 2;
-        const int uvN = (s.flags & SIM_GEOMETRIC) ? (R + 1) * W2 + (R + 2) * W1 + 2 * W1 : 0;
+        const int uvN = geom ? (R + 1) * W2 + (R + 2) * W1 + 2 * W1 : 0;
         float* cofRow[3];
-        cofRow[0] = lds + 2 * plane + max(plane, uvN);
+        cofRow[0] = lds + (polar ? 3 * plane + uvN : 2 * plane + max(plane, uvN));
         cofRow[1] = cofRow[0] + (R + 2);
         cofRow[2] = cofRow[1] + (R + 2);
         // per wavefront: max |u_phi|, |u_theta| of its staged items and max
@@ -459,7 +532,35 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         // forces the checked path (fmaxf would drop a NaN)
         unsigned mp = 0u, mt = 0u;
         auto absbits = [](float v) { return __float_as_uint(v) & 0x7fffffffu; };
-        if (((nP | W) & 3) == 0) {
+        if (polar) {
+            // straight into LDS, every load of the tile in flight at once:
+            // item e of a plane lands at e; 16 bytes each where windows,
+            // half turn and seam are multiples of four columns, else 4
+            auto stage = [&](auto vecTag) __attribute__((always_inline)) {
+                constexpr int V = decltype(vecTag)::value;
+                const int perRow = 2 * win / V, n = plane / V, half = nP >> 1;
+                const unsigned magic = 0xffffffffu / (unsigned)perRow + 1u;  // e / perRow, e < 2^16
+                for (int base = 0; base < n; base += nthr) {
+                    const int e = base + tid;
+                    if (e < n) {
+                        const int r = (int)__umulhi((unsigned)e, magic), c = (e - __mul24(r, perRow)) * V;
+                        int gi = c0 - polarD + c + (c >= win ? half - win : 0);
+                        gi += (gi < 0) ? nP : 0;
+                        gi -= (gi >= nP) ? nP : 0;
+                        const int o = __mul24(rlo + r, nP) + gi;
+                        float* dst = lds + (base + (tid & ~63)) * V;  // the wavefront's; lanes follow in order
+                        load_to_lds<4 * V>(up, dst, o);
+                        load_to_lds<4 * V>(ut, dst + plane, o);
+                        load_to_lds<4 * V>(rh, dst + 2 * plane, o);
+                    }
+                }
+            };
+            if (((nP | W | polarD | (nP >> 1)) & 3) == 0)
+                stage(std::integral_constant<int, 4>{});
+            else
+                stage(std::integral_constant<int, 1>{});
+            __builtin_amdgcn_s_waitcnt(0);
+        } else if (((nP | W) & 3) == 0) {
             // four columns per item: c0 - kEC, SC, nP and SW are multiples of
             // 4, so a float4 never straddles the phi seam and lands 16-byte
             // aligned in LDS
@@ -511,18 +612,20 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
                 mt = max(mt, absbits(b));
             }
         }
-        mp = wave_max(mp);
-        mt = wave_max(mt);
-        mc = wave_max(mc);
-        if ((tid & 63) == 0) {
-            wmax[0][tid >> 6] = mp;
-            wmax[1][tid >> 6] = mt;
-            wmax[2][tid >> 6] = mc;
+        if (!polar) {
+            mp = wave_max(mp);
+            mt = wave_max(mt);
+            mc = wave_max(mc);
+            if ((tid & 63) == 63) {
+                wmax[0][tid >> 6] = mp;
+                wmax[1][tid >> 6] = mt;
+                wmax[2][tid >> 6] = mc;
+            }
         }
         __syncthreads();
         // fast tile: every sample an ordinary bilinear read of the staged block
-        bool fast;
-        {
+        bool fast = false;
+        if (!polar) {
             unsigned m[3] = {0u, 0u, 0u};
 #pragma unroll
             for (int k = 0; k < 3; ++k)
@@ -531,15 +634,14 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
             const float Up = __uint_as_float(m[0]), Ut = __uint_as_float(m[1]);
             const float hmax = __uint_as_float(m[2]);
             // a departure moves at most 2 h max|u| cells
-            fast = (j0 >= kER + 1) && (j0 + R <= nT - kER - 1) && (Up * hmax <= 0.5f * kFastDPhi) &&
-                   (Ut * hT <= 0.5f * kFastDTheta);
+            fast = (Up * hmax <= 0.5f * kFastDPhi) && (Ut * hT <= 0.5f * kFastDTheta);
         }
 
         // one backtrace at node (c, j) of the tile (c from -1, j global): the
         // branch-free staged sampler on fast tiles, the checked one otherwise;
         // ofs = the node's staged offset (j - js) SW + c + kEC, which row walks
         // carry from one row to the next
-        auto nodeAt = [&](auto fastTag, auto nodeTag, int c, int j, float hP, int ofs) -> float {
+        auto nodeAt = [&](auto fastTag, auto nodeTag, int c, int j, float hP, int ofs) __attribute__((always_inline)) -> float {
             constexpr int NK = decltype(nodeTag)::value;
             if constexpr (decltype(fastTag)::value) {
                 return advect_node_fast<NK, NK, SW>(lds, plane, ofs, hP, hT);
@@ -548,15 +650,100 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
                 return advect_node_st<NK, NK, SW>(st, up, ut, src, g, col(c), j, c + kEC, j - js, hP, hT);
             }
         };
-        auto node = [&](auto fastTag, auto nodeTag, int c, int j, float hP) -> float {
+        auto node = [&](auto fastTag, auto nodeTag, int c, int j, float hP) __attribute__((always_inline)) -> float {
             return nodeAt(fastTag, nodeTag, c, j, hP, __mul24(j - js, SW) + c + kEC);
         };
         using KPhi = std::integral_constant<int, K_VPHI>;
         using KTheta = std::integral_constant<int, K_VTHETA>;
         using KRho = std::integral_constant<int, K_CENTERED>;
 
-        if (!(s.flags & SIM_GEOMETRIC)) {
-            auto plain = [&](auto F) {
+        // ---- a polar tile's backtraces, as tasks of 64 columns that the
+        // wavefronts take in turn; the tile's edge columns form tasks of their
+        // own (a task's lanes are nodes of one kind)
+        const int uLo = j0, uHi = min(j0 + R, nT - 1);
+        const int vLo = max(j0 - 1, 0), vHi = min(j0 + R, nT - 2);
+        const bool north = (j0 == 0), south = (uHi == nT - 1);
+        // the rho nodes go first; in tiles clear of the poles their staged
+        // plane then holds U, V, A0, AL (polar tiles keep these apart)
+        float* U = lds + (polar ? 3 : 2) * plane;  // (R+1) x W2: u_phi*, columns c0-1 .. c0+W
+        float* V = U + (R + 1) * W2;               // (R+2) x W1: u_theta*, columns c0-1 .. c0+W-1
+        float* A0 = V + __mul24(R + 2, W1);        // W1: u_theta* of row 0 at the antipodal columns
+        float* AL = A0 + W1;                       // W1: u_theta* of row nT-2 at the antipodal columns
+        if (polar) {
+            PolarStage ps;
+            ps.S = lds;
+            ps.plane = plane;
+            ps.stride = 2 * win;
+            ps.win = win;
+            ps.rlo = rlo;
+            ps.rows[K_VPHI] = ps.rows[K_CENTERED] = min(nT, js + SR) - rlo;
+            ps.rows[K_VTHETA] = min(nT - 1, js + SR) - rlo;
+            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
+            const int v0 = geom ? vLo : j0;
+            const int nUr = geom ? uHi - uLo + 1 : R, nVr = geom ? vHi - vLo + 1 : min(R, nT - 1 - j0);
+            const int nA = geom ? (north ? 1 : 0) + (south ? 1 : 0) : 0;
+            const int wide = W > 64 ? 1 : 0, nc = 1 + wide;  // 64-column chunks of a row
+            const int tR = R * nc, tU = nUr * nc, tV = (nVr + nA) * nc;
+            const int tUe = geom ? (2 * nUr + 63) >> 6 : 0, tVe = geom ? (nVr + nA + 63) >> 6 : 0;
+            bool bad = false;
+            for (int t = wave; t < tR + tU + tUe + tV + tVe; t += kAdvWaves) {
+                int k = t;
+                if (k < tR) {
+                    const int r = k >> wide, c = ln + (wide ? (k & 1) << 6 : 0), j = j0 + r;
+                    if (c < W) {
+                        const float a = advect_node_polar<K_CENTERED>(ps, up, ut, rh, g, col(c), j, c + polarD, 0,
+                                                                      cofRow[0][r + 1], hT);
+                        stf(orhR, (c0 + c) * 4, j * nP * 4, a);
+                        bad |= !isfinite(a);
+                    }
+                    continue;
+                }
+                k -= tR;
+                if (k < tU + tUe) {
+                    int r = k >> wide, c = ln + (wide ? (k & 1) << 6 : 0);
+                    bool on = c < W;
+                    if (k >= tU) {  // columns -1 and W
+                        const int e = ((k - tU) << 6) + ln;
+                        r = e >> 1;
+                        c = (e & 1) ? W : -1;
+                        on = r < nUr;
+                    }
+                    if (on) {
+                        const float a = advect_node_polar<K_VPHI>(ps, up, ut, up, g, col(c), uLo + r, c + polarD, 0,
+                                                                  cofRow[0][r + 1], hT);
+                        if (geom)
+                            U[__mul24(r, W2) + c + 1] = a;
+                        else
+                            stf(oupR, (c0 + c) * 4, (uLo + r) * nP * 4, a);
+                    }
+                    continue;
+                }
+                k -= tU + tUe;
+                // rows nVr and nVr + 1 stand for the antipodal rows (north, then south)
+                int r = k >> wide, c = ln + (wide ? (k & 1) << 6 : 0);
+                bool on = c < W;
+                if (k >= tV) {  // column -1
+                    r = ((k - tV) << 6) + ln;
+                    c = -1;
+                    on = r < nVr + nA;
+                }
+                if (on) {
+                    const bool anti = r >= nVr;
+                    const bool atNorth = anti && north && r == nVr;
+                    const int j = anti ? (atNorth ? 0 : nT - 2) : v0 + r;
+                    int i = col(c) + (anti ? g.half : 0);
+                    i -= (i >= nP) ? nP : 0;
+                    const float a = advect_node_polar<K_VTHETA>(ps, up, ut, ut, g, i, j, c + polarD, anti ? 1 : 0,
+                                                                cofRow[1][j - j0 + 1], hT);
+                    if (geom)
+                        V[(anti ? __mul24(R + 2, W1) + (atNorth ? 0 : W1) : __mul24(r, W1)) + c + 1] = a;
+                    else
+                        stf(outR, (c0 + c) * 4, j * nP * 4, a);
+                }
+            }
+            flag_bad(status, bad);
+        } else if (!geom) {
+            auto plain = [&](auto F) __attribute__((always_inline)) {
                 bool bad = false;
                 for (int idx = tid; idx < R * W; idx += nthr) {
                     const int r = (int)__umulhi((unsigned)idx, mW), c = idx - r * W;
@@ -573,20 +760,13 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
                 plain(std::true_type{});
             else
                 plain(std::false_type{});
+        }
+        if (!geom) {
             __syncthreads();
             continue;
         }
 
-        const int uLo = j0, uHi = min(j0 + R, nT - 1);
-        const int vLo = max(j0 - 1, 0), vHi = min(j0 + R, nT - 2);
-        // the rho nodes go first; their staged plane then holds U, V, A0, AL
-        float* U = lds + 2 * plane;      // (R+1) x W2: u_phi*, columns c0-1 .. c0+W
-        float* V = U + (R + 1) * W2;     // (R+2) x W1: u_theta*, columns c0-1 .. c0+W-1
-        float* A0 = V + (R + 2) * W1;    // W1: u_theta* of row 0 at the antipodal columns
-        float* AL = A0 + W1;             // W1: u_theta* of row nT-2 at the antipodal columns
         float* X = lds;                  // R x W1: cubic roots, over the staged block once it is dead
-        const bool north = (j0 == 0), south = (uHi == nT - 1);
-        const int half = g.half;
         const int nU = (uHi - uLo + 1) * W2, nV = (vHi - vLo + 1) * W1, nR = R * W;
         // One backtrace per item.  Tiles 64 or 128 columns wide map each thread
         // to one tile column (cm) and a run of rows (rm0, rm0 + rmS, ...), with
@@ -605,7 +785,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         const int cm = tid & (kColW - 1), rm0 = __builtin_amdgcn_readfirstlane(tid / kColW);
         const int colB = (c0 + cm) * 4;  // the lane's column in a row of the grid, in bytes
         const int nUr = uHi - uLo + 1, nVr = vHi - vLo + 1;
-        auto advect_all = [&](auto F) {
+        auto advect_all = [&](auto F) __attribute__((always_inline)) {
             if (colMap) {
                 const int dOfs = __mul24(rmS, SW);
                 int ofs = __mul24(j0 + rm0 - js, SW) + cm + kEC;
@@ -656,20 +836,8 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         };
         if (fast)
             advect_all(std::true_type{});
-        else
+        else if (!polar)
             advect_all(std::false_type{});
-        if (north || south) {
-            for (int idx = tid; idx < 2 * W1; idx += nthr) {
-                const bool s0 = idx < W1;
-                if (s0 ? !north : !south) continue;
-                const int c = s0 ? idx : idx - W1;
-                int io = col(c - 1) + half;
-                io -= (io >= nP) ? nP : 0;
-                const int j = s0 ? 0 : nT - 2;
-                const float a = advect_node<K_VTHETA, K_VTHETA>(up, ut, ut, g, io, j, 0.5f * cofPT[j], hT);
-                (s0 ? A0 : AL)[c] = a;
-            }
-        }
         __syncthreads();
 
         // geometricFillKernel, one cell per item: the root x and v' = vbar + G x^2
@@ -677,7 +845,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         // restagger), both into the dead staged block
         const int nG = (uHi - j0 + 1) * W1;
         float* VP = X + (R + 1) * W1;  // (R+1) x W1: v'
-        auto geo = [&](int r, int c) {
+        auto geo = [&](int r, int c) __attribute__((always_inline)) {
             const int idx = r * W1 + c, j = j0 + r;
             const float* Ur = U + (j - uLo) * W2;
             const float ub = 0.5f * (Ur[c] + Ur[c + 1]);
@@ -706,7 +874,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         __syncthreads();
         // assignPhiKernel (rows j0..j0+R-1) and assignThetaKernel (rows
         // j0..uHi-1), columns c0..c0+W-1
-        auto assign = [&](int r, int c) {
+        auto assign = [&](int r, int c) __attribute__((always_inline)) {
             const int o = (j0 + r) * nP + c0 + c, x = r * W1 + c;
             oup[o] = 0.5f * (X[x] + X[x + 1]);
             if (j0 + r < uHi) out[o] = 0.5f * (VP[x + 1] + VP[x + W1 + 1]);
@@ -1992,14 +2160,14 @@ static inline int grid_for(int ntiles, int cap) {
 }
 
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                         int stride, size_t ldsBytes, int gridCap, hipStream_t st) {
+                         int stride, int polarD, size_t ldsBytes, int gridCap, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
     if (stride == adv_stride(64))
         hipLaunchKernelGGL(k_advect<adv_stride(64)>, dim3(grid_for(ntiles, gridCap)), dim3(256),
-                           ldsBytes, st, sims, tiles, ntiles, parity);
+                           ldsBytes, st, sims, tiles, ntiles, parity, polarD);
     else if (stride == adv_stride(128))
         hipLaunchKernelGGL(k_advect<adv_stride(128)>, dim3(grid_for(ntiles, gridCap)), dim3(256),
-                           ldsBytes, st, sims, tiles, ntiles, parity);
+                           ldsBytes, st, sims, tiles, ntiles, parity, polarD);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

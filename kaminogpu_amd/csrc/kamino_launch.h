@@ -19,8 +19,10 @@ constexpr int adv_stride(int W) { return (W <= 64 ? 64 : 128) + 2 * kAdvHaloCols
 // power-of-two size) one slot is left free after every 16 values too.
 constexpr int fft_row_stride(int M, bool padded) { return M + (padded ? M >> 4 : 0) + 4; }
 
+// polarD: columns that polar tiles stage on either side of theirs (PolarStage),
+// a multiple of 4, at most half of every member's nPhi.
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                         int stride, size_t ldsBytes, int gridCap, hipStream_t st);
+                         int stride, int polarD, size_t ldsBytes, int gridCap, hipStream_t st);
 hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                             int gridCap, hipStream_t st);
 // kernel: M where every row FFT of the launch has the same length M = 2^k >= 32

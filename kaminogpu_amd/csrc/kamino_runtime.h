@@ -101,6 +101,7 @@ struct TileLayout {
     size_t advLds = 0, fftLds = 0, fftLds64 = 0, divLds = 0;
     int fftKernel = 0;  // the transform kernels' variant (launch_div_fft)
     int advStride = 0;  // staged row stride of the advection launch
+    int polarD = 0;     // side columns of its polar tiles
 };
 
 // Plans the tiles of n simulations: writes the first min(cap, needed) tiles to

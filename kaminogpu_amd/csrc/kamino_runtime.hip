@@ -63,6 +63,21 @@ static size_t adv_lds(int R, int W, int SW, bool geometric) {
     const size_t uv = geometric ? (size_t)(R + 1) * (W + 2) + (R + 2) * (W + 1) + 2 * (W + 1) : 0;
     return (2 * plane + std::max(plane, uv) + 3 * (size_t)(R + 2) + 3 * (256 / 64)) * sizeof(float);
 }
+// Rows of a band starting within kAdvHaloRows + 1 rows of a pole, or ending
+// there (polar_rows: the bands next to the poles are that tall if R allows).
+constexpr int kPoleRows = kAdvHaloRows + 1;
+static bool polar_bands(int nT, int R) { return R >= kPoleRows && nT > 2 * kPoleRows; }
+// LDS of the polar tiles (k_advect, PolarStage): three planes of the rows they
+// reach and two windows of W columns with D side columns, the advected block
+// beside them, row coefficients and maxima.  The tallest are poleTile rows of
+// the polar bands, or without such bands any R rows.
+static size_t polar_lds(int nT, int R, int poleTile, int W, int D, bool geometric) {
+    const int r = polar_bands(nT, R) ? poleTile : std::min(R, nT);
+    const int rows = std::min(nT, polar_bands(nT, R) ? std::min(kPoleRows, r + kAdvHaloRows) + kAdvHaloRows
+                                                     : r + 2 * kAdvHaloRows);
+    const size_t uv = geometric ? (size_t)(r + 1) * (W + 2) + (r + 2) * (W + 1) + 2 * (W + 1) : 0;
+    return ((size_t)3 * rows * 2 * (W + 2 * D) + uv + 3 * (size_t)(r + 2) + 3 * (256 / 64)) * sizeof(float);
+}
 // The elementary radices and items per lane of each kind of FFT pass.
 struct Radices {
     int R1, R2, I;
@@ -634,7 +649,14 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
                 set_tile_cols(sims[s], advCols[s]);
             }
     L.advStride = adv_stride(wide && !narrow ? kAdvMaxCols : kAdvMaxCols / 2);
-    shrink_until_busy(plans, n, advRows, minTiles, advCols);
+    // A launch of few tiles runs them all at once and lasts as long as its
+    // slowest: the polar bands, whose samples take the pole rules, go out as
+    // tiles of one row there (a 256 x 512 step 25.5 us with four-row ones, 24.4
+    // with two, 23.7 with one; from 512 x 1024 on the same or, with few rows
+    // left to the other tiles, 0.5 us slower).
+    const int advTiles = shrink_until_busy(plans, n, advRows, minTiles, advCols);
+    const bool few = advTiles <= 4 * device_cus();
+    const int poleTile = few ? 1 : kPoleRows;
     shrink_until_busy(plans, n, fftRows, minTiles, nullptr);
     // advection tiles, in batch order (tallest simulations first); the last
     // column tile of a row band overlaps its neighbour instead of running short.
@@ -643,18 +665,17 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     // are exactly that tall when the tile height allows, and every band between
     // them can take the fast one; the last inner band may be shorter.
     L.advOff = 0;
-    constexpr int kPoleRows = kAdvHaloRows + 1;
     for (int s = 0; s < n; ++s) {
         const Plan& p = plans[s];
         const int W = advCols[s], R = advRows[s];
-        const bool polar = R >= kPoleRows && p.nT > 2 * kPoleRows;
+        const bool polar = polar_bands(p.nT, R);
         for (int j = 0, rows; j < p.nT; j += rows) {
             if (!polar)
                 rows = std::min(R, p.nT - j);
-            else if (j == 0)
-                rows = kPoleRows;
+            else if (j < kPoleRows)
+                rows = std::min(poleTile, kPoleRows - j);
             else if (j >= p.nT - kPoleRows)
-                rows = p.nT - j;
+                rows = std::min(poleTile, p.nT - j);
             else
                 rows = std::min(R, p.nT - kPoleRows - j);
             for (int c = 0; c < p.nP; c += W) put(Tile{s, j, rows, std::min(c, p.nP - W)});
@@ -662,6 +683,29 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
         L.advLds = std::max(L.advLds, adv_lds(advRows[s], W, L.advStride, (sims[s].flags & SIM_GEOMETRIC) != 0));
     }
     L.nAdv = cnt;
+    // The polar tiles' side columns: what a flow of speed 1.25 moves in the row
+    // next to a pole, as far as LDS allows.  A launch of few tiles gives a CU
+    // 40 KiB per tile without running fewer at once; one of many keeps to its
+    // other tiles' LDS, or a seventh of a CU's.
+    const size_t room = few ? 40 * 1024 : std::max(L.advLds, (size_t)kLdsMax / 7);
+    int most = 4;
+    for (int s = 0; s < n; ++s) {
+        const double h = kPi / plans[s].nT;
+        const double cells = 1.25 * sims[s].cofTheta / std::sin(0.5 * h) + 3.0;
+        most = std::max(most, (int)std::min(cells, 64.0));
+    }
+    for (int s = 0; s < n; ++s) most = std::min(most, plans[s].nP / 2);
+    for (L.polarD = (most + 3) & ~3; L.polarD > 4; L.polarD -= 4) {
+        bool ok = true;
+        for (int s = 0; s < n && ok; ++s)
+            ok = L.polarD <= plans[s].nP / 2 &&
+                 polar_lds(plans[s].nT, advRows[s], poleTile, advCols[s], L.polarD,
+                           (sims[s].flags & SIM_GEOMETRIC) != 0) <= room;
+        if (ok) break;
+    }
+    for (int s = 0; s < n; ++s)
+        L.advLds = std::max(L.advLds, polar_lds(plans[s].nT, advRows[s], poleTile, advCols[s], L.polarD,
+                                                (sims[s].flags & SIM_GEOMETRIC) != 0));
     // FFT tiles: simulations with the FP32 pressure first, then those with the
     // FP64 pressure, whose inverse transform is a launch of its own (FP64 rows
     // in LDS: their tiles hold as many rows as fit)
@@ -773,7 +817,7 @@ int launch_step(const SimDesc* dSims, const Tile* dTiles, const TileLayout& L, i
     }
     if (phases & KAM_PHASE_ADVECT) {
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT], st));
-        KAM_HIP(launch_advect(dSims, dTiles + L.advOff, L.nAdv, p, L.advStride, L.advLds, kGridCap, st));
+        KAM_HIP(launch_advect(dSims, dTiles + L.advOff, L.nAdv, p, L.advStride, L.polarD, L.advLds, kGridCap, st));
         KAM_HIP(launch_particles(dSims, dTiles + L.partOff, L.nPart, p, kGridCap, st));
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT + 1], st));
         p ^= 1;
