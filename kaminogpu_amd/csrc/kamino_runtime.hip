@@ -137,7 +137,7 @@ static void plan_pow2(FftPlan& pl) {
         add_pass(pl, M, pass_kind(4, R / 4, (M / R + P::lanes - 1) / P::lanes), Ls, tw0);
     }
 }
-static void plan_fft(int M, const int* fac, int nfac, FftPlan& best) {
+static void search_fft(int M, const int* fac, int nfac, FftPlan& best) {
     switch (M) {
 #define KAM_CASE(m) \
     case m: plan_pow2<m>(best); return;
@@ -175,6 +175,19 @@ static void plan_fft(int M, const int* fac, int nfac, FftPlan& best) {
             }
         }
     }
+}
+// The plan of M, searched for once (a rebuild of an engine's batch plans every
+// member; the search takes some 50 us).
+static std::mutex g_fft_mu;
+static std::map<int, FftPlan> g_fft;
+static void plan_fft(int M, const int* fac, int nfac, FftPlan& plan) {
+    std::lock_guard<std::mutex> lk(g_fft_mu);
+    auto it = g_fft.find(M);
+    if (it == g_fft.end()) {
+        it = g_fft.emplace(M, FftPlan()).first;
+        search_fft(M, fac, nfac, it->second);
+    }
+    plan = it->second;
 }
 // LDS row stride of a transform row in complex values
 static int fft_stride(int M) { return fft_row_stride(M, (M & (M - 1)) == 0 && M >= 64); }
