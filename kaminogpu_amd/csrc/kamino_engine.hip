@@ -31,6 +31,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "kamino_launch.h"
 #include "kamino_runtime.h"
 
 namespace kam {
@@ -313,10 +314,11 @@ int retire(kam_engine* e, Request& r, int state) {
         r.hostBytes = 3 * N * sizeof(float);
         r.host = e->pinned.get(r.hostBytes);
         if (!r.host) return set_err(KAM_ENOMEM, "pinned host allocation failed");
-        float* h = static_cast<float*>(r.host);
-        for (int f = 0; f < 3; ++f)
-            KAM_HIP(hipMemcpyAsync(h + f * N, r.desc.state[e->parity][f], N * sizeof(float),
-                                   hipMemcpyDeviceToHost, e->stream));
+        // the three fields lie in a row; a kernel writes them to the pinned copy
+        const Ranges out = {{r.host, nullptr, nullptr, nullptr, nullptr, nullptr},
+                            {r.desc.state[e->parity][0], nullptr, nullptr, nullptr, nullptr, nullptr},
+                            {(int64_t)(3 * N), 0, 0, 0, 0, 0}};
+        KAM_HIP(launch_ranges(out, e->stream));
         KAM_HIP(hipEventCreateWithFlags(&r.copied, hipEventDisableTiming));
         KAM_HIP(hipEventRecord(r.copied, e->stream));
         r.copying = true;

@@ -2173,6 +2173,36 @@ hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int
     return hipGetLastError();
 }
 
+// Moves ranges with vector accesses (which also works where a caller captures
+// the stream into a graph): 16 bytes at a time where a range's pointers allow
+// it (the fields of odd sizes lie 4 n_theta^2 mod 16 bytes apart, and callers'
+// slices anywhere), else four.
+__global__ __launch_bounds__(256) void k_ranges(Ranges a) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int r = 0; r < kMaxRanges; ++r) {
+        unsigned* const d = static_cast<unsigned*>(a.dst[r]);
+        const unsigned* const s = static_cast<const unsigned*>(a.src[r]);
+        const int64_t n = a.n[r];
+        int64_t i = first;
+        if (((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(s)) & 15) == 0) {
+            uint4* const d4 = reinterpret_cast<uint4*>(d);
+            const uint4* const s4 = reinterpret_cast<const uint4*>(s);
+            for (; i < n / 4; i += stride) d4[i] = s ? s4[i] : make_uint4(0, 0, 0, 0);
+            i = (n & ~(int64_t)3) + first;
+        }
+        for (; i < n; i += stride) d[i] = s ? s[i] : 0u;
+    }
+}
+
+hipError_t launch_ranges(const Ranges& a, hipStream_t st) {
+    int64_t total = 0;
+    for (int r = 0; r < kMaxRanges; ++r) total += a.n[r];
+    // four values a thread, at most four workgroups a CU
+    const int64_t blocks = (total + 4 * 256 - 1) / (4 * 256);
+    hipLaunchKernelGGL(k_ranges, dim3((unsigned)(blocks < 1024 ? (blocks > 0 ? blocks : 1) : 1024)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                             int gridCap, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;

@@ -56,6 +56,21 @@ hipError_t launch_dft_pressure(const SimDesc* sims, const Tile* gemmTiles, int n
                                hipStream_t st);
 constexpr int kDftTileRows = 64, kDftTileCols = 128, kDftChunk = 32;
 
+// Ranges of 4-byte values to copy (src given) or to clear (src null) by one
+// launch; the kernel reads and writes them, so they are this device's memory or
+// pinned host memory.  A runtime copy between pinned and device memory goes to a
+// copy engine and back, 10 us and more in the stream for a few kilobytes: with
+// an engine's tables and finished fields moved by this kernel, 48 steps of 64
+// spheres of 32 to 256 rows with eight retirements take 3.5 to 4.2 ms instead of
+// 5.1.  (A copy stream beside the engine's for the finished fields: the same.)
+constexpr int kMaxRanges = 6;
+struct Ranges {
+    void* dst[kMaxRanges];
+    const void* src[kMaxRanges];
+    int64_t n[kMaxRanges];  // values
+};
+hipError_t launch_ranges(const Ranges& a, hipStream_t st);
+
 // Raises the dynamic-LDS limit of every step kernel to `bytes` (call once).
 hipError_t configure_kernels(size_t bytes);
 

@@ -79,47 +79,6 @@ struct Stage {
 };
 Stage g_stage;
 
-// Float ranges to copy (src given) or to clear (src null), all by one launch.
-constexpr int kMaxRanges = 6;
-struct Ranges {
-    float* dst[kMaxRanges];
-    const float* src[kMaxRanges];
-    int n[kMaxRanges];
-};
-
-// Moves the ranges with vector stores (which also works where a caller captures
-// the stream into a graph).  A range whose pointers are 16-byte aligned goes
-// four values at a time; the fields of odd sizes, 4 n_theta^2 (mod 16) bytes
-// apart, and callers' slices at odd addresses go one value at a time.  One
-// launch on either side of the steps in place of three copies and a clear
-// before them and three copies after, each about 2 us of a call (one step of
-// 32 x 64: 38.3 -> 29.7 us a call; eight of 256 x 512: 254 -> 246 us).
-__global__ __launch_bounds__(256) void k_ranges(Ranges a) {
-    const int stride = gridDim.x * blockDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int r = 0; r < kMaxRanges; ++r) {
-        float* const d = a.dst[r];
-        const float* const s = a.src[r];
-        const int n = a.n[r];
-        int i = first;
-        if (((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(s)) & 15) == 0) {
-            float4* const d4 = reinterpret_cast<float4*>(d);
-            const float4* const s4 = reinterpret_cast<const float4*>(s);
-            for (; i < n / 4; i += stride) d4[i] = s ? s4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-            i = (n & ~3) + first;
-        }
-        for (; i < n; i += stride) d[i] = s ? s[i] : 0.f;
-    }
-}
-
-hipError_t launch_ranges(const Ranges& a, hipStream_t st) {
-    int64_t total = 0;
-    for (int r = 0; r < kMaxRanges; ++r) total += a.n[r];
-    // four values a thread, at most four workgroups a CU
-    const int64_t blocks = (total + 4 * 256 - 1) / (4 * 256);
-    hipLaunchKernelGGL(k_ranges, dim3((unsigned)(blocks < 1024 ? (blocks > 0 ? blocks : 1) : 1024)), dim3(256), 0, st, a);
-    return hipGetLastError();
-}
-
 // Whether [p, p + bytes) lies within one allocation of `device`'s own memory,
 // which a kernel on it may read and write.
 bool own_memory(const void* p, size_t bytes, int device) {
@@ -234,21 +193,24 @@ extern "C" int kam_sim_step_noalloc(const kam_sim_desc* d, float* u_phi, float* 
     // and, without rho, the density read as zero.  One launch moves fields in
     // this device's memory; any others (host-mapped, another device's, or
     // past their allocation) go through the runtime's copies, which know how to
-    // reach them or refuse them.
+    // reach them or refuse them.  One launch on either side of the steps in
+    // place of three copies and a clear before them and three copies after,
+    // each about 2 us of a call (one step of 32 x 64: 38.3 -> 29.7 us a call;
+    // eight of 256 x 512: 254 -> 246 us).
     const bool direct = own_memory(u_phi, N * sizeof(float), d->device) &&
                         own_memory(u_theta, Nt * sizeof(float), d->device) &&
                         (!rho || own_memory(rho, N * sizeof(float), d->device));
     Ranges in = {{sd.state[0][F_UTHETA] + Nt, sd.state[1][F_UTHETA] + Nt, reinterpret_cast<float*>(sd.status),
                   sd.state[0][F_RHO], nullptr, nullptr},
                  {nullptr, nullptr, nullptr, rho, nullptr, nullptr},
-                 {nP, nP, 1, (int)N, 0, 0}};
+                 {nP, nP, 1, (int64_t)N, 0, 0}};
     if (direct) {
         in.dst[4] = sd.state[0][F_UPHI];
         in.src[4] = u_phi;
-        in.n[4] = (int)N;
+        in.n[4] = (int64_t)N;
         in.dst[5] = sd.state[0][F_UTHETA];
         in.src[5] = u_theta;
-        in.n[5] = (int)Nt;
+        in.n[5] = (int64_t)Nt;
     } else {
         KAM_HIP(hipMemcpyAsync(sd.state[0][F_UPHI], u_phi, N * sizeof(float), hipMemcpyDeviceToDevice, st));
         KAM_HIP(hipMemcpyAsync(sd.state[0][F_UTHETA], u_theta, Nt * sizeof(float), hipMemcpyDeviceToDevice, st));
@@ -270,7 +232,7 @@ extern "C" int kam_sim_step_noalloc(const kam_sim_desc* d, float* u_phi, float* 
     if (direct) {
         const Ranges out = {{u_phi, u_theta, rho, nullptr, nullptr, nullptr},
                             {sd.state[p][F_UPHI], sd.state[p][F_UTHETA], sd.state[p][F_RHO], nullptr, nullptr, nullptr},
-                            {(int)N, (int)Nt, rho ? (int)N : 0, 0, 0, 0}};
+                            {(int64_t)N, (int64_t)Nt, rho ? (int64_t)N : 0, 0, 0, 0}};
         KAM_HIP(launch_ranges(out, st));
         return KAM_OK;
     }

@@ -877,10 +877,13 @@ int DeviceBatch::build(const std::vector<SimDesc>& simsIn, const std::vector<Pla
     const size_t sb = sims.size() * sizeof(SimDesc), tb = hTiles_.size() * sizeof(Tile);
     std::memcpy(stage, sims.data(), sb);
     std::memcpy(stage + capSims_ * sizeof(SimDesc), hTiles_.data(), tb);
-    if (sb) KAM_HIP(hipMemcpyAsync(dSims_, stage, sb, hipMemcpyHostToDevice, st));
-    if (tb)
-        KAM_HIP(hipMemcpyAsync(dTiles_, stage + capSims_ * sizeof(SimDesc), tb,
-                               hipMemcpyHostToDevice, st));
+    static_assert(sizeof(SimDesc) % 16 == 0 && sizeof(Tile) % 4 == 0, "moved in 4- or 16-byte values");
+    if (sb || tb) {
+        const Ranges up = {{dSims_, dTiles_, nullptr, nullptr, nullptr, nullptr},
+                           {stage, stage + capSims_ * sizeof(SimDesc), nullptr, nullptr, nullptr, nullptr},
+                           {(int64_t)(sb / 4), (int64_t)(tb / 4), 0, 0, 0, 0}};
+        KAM_HIP(launch_ranges(up, st));
+    }
     KAM_HIP(hipEventRecord(uploaded_[cur_], st));
     return KAM_OK;
 }
