@@ -1539,12 +1539,23 @@ __device__ __forceinline__ T shfl_grp(T v, int srcLaneInGroup, int laneBase) {
 // write-back.
 constexpr int kTriBatch = 4;  // float4 spectrum loads per thread in flight while staging
 
-template <int L, int KMAX, bool RESID, typename T>
-__device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const Tile& tile,
-                                         int parity, float2* zsp, double* csp, double* ssp,
-                                         float* fsp) {
-    constexpr int G = 256 / L;  // modes per block
-    (void)G;
+// A block is one dependent chain (stage, Thomas, log2 L reductions, back
+// substitution, write back) on few waves, so what bounds it on a single sphere
+// is its instruction count, about 5 cycles each per wave; large batches are
+// bound by the spectrum's 16 bytes per cell (268 MB in 29.9 us, 9 TB/s through
+// the caches, at 128 spheres of 256).  Hence no slot of a staging batch that no
+// thread needs, one reciprocal per reduction, shared by shuffle with both
+// neighbours, and no selects at the ends of a group.
+//
+// FULL: the tile holds 256 / L modes of a simulation with exactly L KMAX rows,
+// so the row count per lane is a constant: every row guard folds away, rows
+// split into (lane, row) by shifts and pairs by constants.  A step of one
+// sphere, before these cuts and after: 23.8 -> 21.8 us at nTheta 256,
+// 62.3 -> 59.8 at 1024, 175 -> 167 at 2048; of 405, never full, 33.4 -> 33.3.
+template <int L, int KMAX, bool RESID, typename T, bool FULL>
+__device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, const Tile& tile,
+                                            int parity, float2* zsp, double* csp, double* ssp,
+                                            float* fsp) {
     // SF: the subtraction-free pivots of the FP32 elimination, from FP32 row
     // tables; the FP64 row terms are staged for the FP64 elimination and for
     // the residual report
@@ -1565,69 +1576,25 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
     const int base = wl - l;             // first wavefront lane of this group
     {
         const SimDesc& s = sims[tile.sim];
-        const int nT = s.nTheta;
-        const bool p64 = (s.flags & SIM_P64) != 0;
-        double2* __restrict__ spec64 = reinterpret_cast<double2*>(s.state[parity ^ 1][0]);
-        const bool active = g < tile.rows;
+        const int nT = FULL ? L * KMAX : s.nTheta, Ms = FULL ? nT : s.M;
+        const bool p64 = !SF;  // the FP64 elimination serves the FP64 pressure alone
+        const Rsrc spec64R = make_rsrc(s.state[parity ^ 1][0], p64 ? 4 * Ms * nT : 0);
+        const bool active = FULL || g < tile.rows;
         const int n = tile.row0 + (active ? g : 0);
-        const int K = (nT + L - 1) / L;
+        const int rows = FULL ? 256 / L : tile.rows;  // the tile's modes
+        const int K = FULL ? KMAX : (nT + L - 1) / L;
         // i / K and e / nT as multiply-high (exact for dividends below 2^16):
         // ceil(2^32 / K) in its 32-bit form (K = 1, whose multiplier 2^32 does
         // not fit, is taken apart), and e / nT = 2e / nPhi
-        const unsigned magicK = (K == 1) ? 0u : 0xffffffffu / (unsigned)K + 1u;
+        const unsigned magicK = (FULL || K == 1) ? 0u : 0xffffffffu / (unsigned)K + 1u;
         auto split = [&](int i, int& li, int& ki) {
-            li = (K == 1) ? i : (int)__umulhi((unsigned)i, magicK);
+            li = FULL ? i / KMAX : ((K == 1) ? i : (int)__umulhi((unsigned)i, magicK));
             ki = i - li * K;
         };
         const int r0 = l * K;
-        int cnt = nT - r0;
-        cnt = cnt < 0 ? 0 : (cnt > K ? K : cnt);
-        if (!active) cnt = 0;
-        // staging: a thread's loads of a batch all go out before its first
-        // LDS write; reads past the tables or the spectrum return 0 and are
-        // not kept
-        if constexpr (kStage64) {
-            const Rsrc rowR = make_rsrc(reinterpret_cast<const float*>(s.rowd), 2 * RD_COUNT * nT);
-            for (int i0 = tid; i0 < nT; i0 += 4 * 256) {
-                double c[4], v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    c[q] = ldd(rowR, RD_COT2H * nT + i0 + q * 256);
-                    v[q] = ldd(rowR, RD_INVSIN2 * nT + i0 + q * 256);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int i = i0 + q * 256;
-                    if (i >= nT) break;
-                    int li, ki;
-                    split(i, li, ki);
-                    cs(ki, li) = c[q];
-                    ss(ki, li) = v[q];
-                }
-            }
-        }
-        if constexpr (SF) {
-            const Rsrc rowF = make_rsrc(s.rowf, RT_COUNT * nT);
-            for (int i0 = tid; i0 < nT; i0 += 4 * 256) {
-                float a[4], c[4], v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    a[q] = ldf(rowF, RT_TRIA * nT + i0 + q * 256);
-                    c[q] = ldf(rowF, RT_TRIC * nT + i0 + q * 256);
-                    v[q] = ldf(rowF, RT_TRIS * nT + i0 + q * 256);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int i = i0 + q * 256;
-                    if (i >= nT) break;
-                    int li, ki;
-                    split(i, li, ki);
-                    fa(ki, li) = a[q];
-                    fc(ki, li) = c[q];
-                    fs(ki, li) = v[q];
-                }
-            }
-        }
+        int rowsLeft = nT - r0;
+        rowsLeft = rowsLeft < 0 ? 0 : (rowsLeft > K ? K : rowsLeft);
+        const int cnt = FULL ? KMAX : (active ? rowsLeft : 0);  // this lane's rows
         // The tile's entries in spectrum order (spec_index): block by block of
         // kSpecRows rows, in each the tile's modes as runs of kSpecRows rows.
         // Pair p of the tile (two entries, one float4) is mode row0 + g, rows
@@ -1635,12 +1602,12 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
         // g = w / kHalf, i = kSpecRows b + 2 (w % kHalf), at float2 offset
         // kSpecRows (b M + row0) + 2 w (even, so float4-aligned).  Rows past
         // nTheta are padding and are skipped.
-        const Rsrc specR = make_rsrc(s.spec, 2 * s.M * spec_rows(nT));
+        const Rsrc specR = make_rsrc(s.spec, 2 * Ms * spec_rows(nT));
         constexpr int kHalf = kSpecRows / 2;  // pairs per mode in a block
-        const int pairN = kHalf * tile.rows, nPairs = tile.rows * (spec_rows(nT) / 2), Ms = s.M;
-        const unsigned magicB = 0xffffffffu / (unsigned)pairN + 1u;  // p / pairN, p < 2^16, pairN >= 2
+        const int pairN = kHalf * rows, nPairs = rows * (spec_rows(nT) / 2);
+        const unsigned magicB = FULL ? 0u : 0xffffffffu / (unsigned)pairN + 1u;  // p / pairN, p < 2^16, pairN >= 2
         auto pair = [&](int p, int& g, int& i) -> int {
-            const int b = (int)__umulhi((unsigned)p, magicB);
+            const int b = FULL ? p / pairN : (int)__umulhi((unsigned)p, magicB);
             const int w = p - b * pairN;
             g = w / kHalf;
             i = kSpecRows * b + 2 * (w % kHalf);
@@ -1653,32 +1620,92 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
                 ++li;
             }
         };
-        for (int p0 = tid; p0 < nPairs; p0 += 256 * kTriBatch) {
-            float4 v[kTriBatch];
-            int gq[kTriBatch], iq[kTriBatch];
+        // staging: a thread's loads of a batch all go out before its first LDS
+        // write, the first batch's before the tables' too; reads past the
+        // tables or the spectrum return 0 and are not kept
+        float4 v[kTriBatch];
+        auto load = [&](int base) {
 #pragma unroll
             for (int q = 0; q < kTriBatch; ++q) {
-                const int p = p0 + 256 * q;
-                const int a = pair(p, gq[q], iq[q]);
+                if (base + 256 * q >= nPairs) break;
+                const int p = base + 256 * q + tid;
+                int gq, iq;
+                const int a = pair(p, gq, iq);
                 v[q] = ldf4(specR, p < nPairs ? 2 * a : -1);  // pairs past the tile read as 0, unused
             }
+        };
+        load(0);
+        if constexpr (kStage64) {
+            const Rsrc rowR = make_rsrc(reinterpret_cast<const float*>(s.rowd), 2 * RD_COUNT * nT);
+            for (int base = 0; base < nT; base += 4 * 256) {
+                const int i0 = base + tid;
+                double c[4], v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (base + q * 256 >= nT) break;  // no thread needs the slot
+                    c[q] = ldd(rowR, RD_COT2H * nT + i0 + q * 256);
+                    v[q] = ldd(rowR, RD_INVSIN2 * nT + i0 + q * 256);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (base + q * 256 >= nT) break;
+                    const int i = i0 + q * 256;
+                    if (i >= nT) break;
+                    int li, ki;
+                    split(i, li, ki);
+                    cs(ki, li) = c[q];
+                    ss(ki, li) = v[q];
+                }
+            }
+        }
+        if constexpr (SF) {
+            const Rsrc rowF = make_rsrc(s.rowf, RT_COUNT * nT);
+            for (int base = 0; base < nT; base += 4 * 256) {
+                const int i0 = base + tid;
+                float a[4], c[4], v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (base + q * 256 >= nT) break;  // no thread needs the slot
+                    a[q] = ldf(rowF, RT_TRIA * nT + i0 + q * 256);
+                    c[q] = ldf(rowF, RT_TRIC * nT + i0 + q * 256);
+                    v[q] = ldf(rowF, RT_TRIS * nT + i0 + q * 256);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (base + q * 256 >= nT) break;
+                    const int i = i0 + q * 256;
+                    if (i >= nT) break;
+                    int li, ki;
+                    split(i, li, ki);
+                    fa(ki, li) = a[q];
+                    fc(ki, li) = c[q];
+                    fs(ki, li) = v[q];
+                }
+            }
+        }
+        for (int base = 0; base < nPairs; base += 256 * kTriBatch) {
+            if (base > 0) load(base);
 #pragma unroll
             for (int q = 0; q < kTriBatch; ++q) {
-                if (p0 + 256 * q < nPairs && iq[q] < nT) {
+                if (base + 256 * q >= nPairs) break;
+                const int p = base + 256 * q + tid;
+                int gq, iq;
+                pair(p, gq, iq);
+                if ((FULL && nPairs % 256 == 0) || (p < nPairs && iq < nT)) {
                     int li, ki;
-                    split(iq[q], li, ki);
-                    zs(gq[q], ki, li) = make_float2(v[q].x, v[q].y);
-                    if (iq[q] + 1 < nT) {
+                    split(iq, li, ki);
+                    zs(gq, ki, li) = make_float2(v[q].x, v[q].y);
+                    if (FULL || iq + 1 < nT) {
                         step_row(li, ki);
-                        zs(gq[q], ki, li) = make_float2(v[q].z, v[q].w);
+                        zs(gq, ki, li) = make_float2(v[q].z, v[q].w);
                     }
                 }
             }
         }
         __syncthreads();
-        const double h2 = s.invH2;
-        const double nn = (n == 0) ? (double)s.M * (double)s.M : (double)n * (double)n;
-        const float nnf = (float)nn;  // exact: n^2 <= 2^22
+        const double h2 = kStage64 ? s.invH2 : 0.0;
+        const float nf = (float)(n == 0 ? Ms : n), nnf = nf * nf;  // exact: n^2 <= 2^22
+        const double nn = (double)nnf;
         // row i = r0 + k of this lane, a x_{i-1} + b x_i + c x_{i+1} = f, in FP64
         // (the pole rows folded, KaminoSolver.cu:117-163)
         auto coef = [&](int k, double& a, double& b, double& c) {
@@ -1700,13 +1727,7 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
         // dropped: its slot's real part) into (xr, xi), in T: Thomas within
         // the lane, then parallel cyclic reduction of the lanes' last
         // unknowns.
-        // The solve, from the lanes' Thomas passes to the solution's staging
-        // for the write-back, for a row count per lane `cntArg`; a block whose
-        // every lane holds KMAX rows (all its modes active, nTheta = L KMAX)
-        // takes it with the count as a constant, so every row guard folds away.
         T xr[KMAX], xi[KMAX];
-        auto solve = [&](auto cntArg) {
-        const int cnt = cntArg;
         {
             T al[KMAX], ga[KMAX], dr[KMAX], di[KMAX];
 #pragma unroll
@@ -1806,30 +1827,20 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
             // parallel cyclic reduction across the L lanes of the group
 #pragma unroll
             for (int st = 1; st < L; st <<= 1) {
+                // a lane without a neighbour on one side reads itself: its
+                // coupling there, A or C, is 0 (the pole rows have none, and
+                // every reduction keeps it so), and so is what it adds
                 const int lm = l - st, lp = l + st;
                 const int sm = lm >= 0 ? lm : l, sp = lp < L ? lp : l;
-                T Am = shfl_grp<L>(A, sm, base), Bm = shfl_grp<L>(B, sm, base);
-                T Dmr = shfl_grp<L>(Dr, sm, base), Dmi = shfl_grp<L>(Di, sm, base);
-                T Bp = shfl_grp<L>(B, sp, base), Cp = shfl_grp<L>(C, sp, base);
-                T Dpr = shfl_grp<L>(Dr, sp, base), Dpi = shfl_grp<L>(Di, sp, base);
+                const T rB = rcpT(B);
+                const T Am = shfl_grp<L>(A, sm, base), rm = shfl_grp<L>(rB, sm, base);
+                const T Dmr = shfl_grp<L>(Dr, sm, base), Dmi = shfl_grp<L>(Di, sm, base);
+                const T rp = shfl_grp<L>(rB, sp, base), Cp = shfl_grp<L>(C, sp, base);
+                const T Dpr = shfl_grp<L>(Dr, sp, base), Dpi = shfl_grp<L>(Di, sp, base);
                 // SF: the neighbours' excesses; else their other couplings
-                T Xm = SF ? shfl_grp<L>(E, sm, base) : shfl_grp<L>(C, sm, base);
-                T Xp = SF ? shfl_grp<L>(E, sp, base) : shfl_grp<L>(A, sp, base);
-                if (lm < 0) {
-                    Am = T(0);
-                    Bm = T(1);
-                    Dmr = T(0);
-                    Dmi = T(0);
-                    Xm = SF ? T(1) : T(0);
-                }
-                if (lp >= L) {
-                    Bp = T(1);
-                    Cp = T(0);
-                    Dpr = T(0);
-                    Dpi = T(0);
-                    Xp = SF ? T(1) : T(0);
-                }
-                const T k1 = A * rcpT(Bm), k2 = C * rcpT(Bp);
+                const T Xm = SF ? shfl_grp<L>(E, sm, base) : shfl_grp<L>(C, sm, base);
+                const T Xp = SF ? shfl_grp<L>(E, sp, base) : shfl_grp<L>(A, sp, base);
+                const T k1 = A * rm, k2 = C * rp;
                 const T nA = -Am * k1, nC = -Cp * k2;
                 T nB;
                 if constexpr (SF) {
@@ -1916,39 +1927,43 @@ __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const
 #pragma unroll
         for (int k = 0; k < KMAX; ++k) {
             if (k < cnt) {
-                if (p64)
-                    spec64[(size_t)n * nT + r0 + k] = make_double2((n == 0) ? 0.0 : (double)xr[k], (double)xi[k]);
+                if constexpr (!SF)
+                    std2(spec64R, n * nT + r0 + k, make_double2((n == 0) ? 0.0 : (double)xr[k], (double)xi[k]));
                 else
                     zs(g, k, l) = make_float2((n == 0) ? 0.f : (float)xr[k], (float)xi[k]);
             }
         }
-        };
-        if (tile.rows == 256 / L && nT == L * KMAX)
-            solve(std::integral_constant<int, KMAX>{});
-        else
-            solve(cnt);
         __syncthreads();
         if (p64) return;  // the solution is already stored (uniform over the block)
         // write-back in spectrum order, pairs as float4 where both rows are real
-        float* __restrict__ spw = s.spec;
-        for (int p = tid; p < nPairs; p += 256) {
+        for (int base = 0; base < nPairs; base += 256) {
+            const int p = base + tid;
+            if (!(FULL && nPairs % 256 == 0) && p >= nPairs) break;
             int g, i;
             const int a = pair(p, g, i);
-            if (i >= nT) continue;
+            if (!FULL && i >= nT) continue;
             int li, ki;
             split(i, li, ki);
             const float2 x = zs(g, ki, li);
-            if (i + 1 < nT) {
+            if (FULL || i + 1 < nT) {
                 step_row(li, ki);
                 const float2 y = zs(g, ki, li);
-                *reinterpret_cast<float4*>(spw + 2 * (size_t)a) = make_float4(x.x, x.y, y.x, y.y);
+                stf4(specR, 2 * a, make_float4(x.x, x.y, y.x, y.y));
             } else {
-                *reinterpret_cast<float2*>(spw + 2 * (size_t)a) = x;
+                stf2(specR, 2 * a, x);
             }
         }
     }
 }
 
+template <int L, int KMAX, bool RESID, typename T>
+__device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const Tile& tile, int parity, float2* zsp,
+                                         double* csp, double* ssp, float* fsp) {
+    if (tile.rows == 256 / L && sims[tile.sim].nTheta == L * KMAX)
+        tri_tile_as<L, KMAX, RESID, T, true>(sims, tile, parity, zsp, csp, ssp, fsp);
+    else
+        tri_tile_as<L, KMAX, RESID, T, false>(sims, tile, parity, zsp, csp, ssp, fsp);
+}
 
 template <int L, int KMAX, bool RESID, typename T>
 __global__ __launch_bounds__(256) void k_tridiag(const SimDesc* __restrict__ sims,
