@@ -901,10 +901,18 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
 // by the u_phi and u_theta samplers; no phi motion where R sin(theta) <= 1e-7;
 // then validateCoord.  The fold keeps the reference's arithmetic: FP32
 // positions, the 2 pi and pi constants and the remainder in FP64.  A tile is
-// a run of particles of one simulation; each thread moves one at a time.
+// a run of particles of one simulation.
+//
+// What bounds it is the gathers, a cache line per lane and load, and below a
+// few thousand waves their latency.  So the two values a row of a sample needs
+// come as one load, all of an ordinary particle's samples are in flight
+// together, and tiles are short (kPartTile).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void validate_coord(float& phi, float& theta) {
     constexpr double k2Pi = 6.28318530717958647692, kPiD = 3.14159265358979323846;
+    // within both periods (both quotients below 1 also once rounded) the
+    // arithmetic below returns its arguments
+    if (theta >= 0.f && theta <= 3.14f && phi >= 0.f && phi <= 6.283f) return;
     theta = (float)((double)theta - (double)(int)floorf((float)((double)theta / k2Pi)) * k2Pi);
     if ((double)theta > kPiD) {
         theta = (float)(k2Pi - (double)theta);
@@ -920,33 +928,69 @@ __device__ __forceinline__ void validate_coord(float& phi, float& theta) {
 __global__ __launch_bounds__(256) void k_particles(const SimDesc* __restrict__ sims,
                                                    const Tile* __restrict__ tiles, int ntiles,
                                                    int parity) {
-    for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles) {
-        const Tile tile = tiles[t];
-        const SimDesc& s = sims[tile.sim];
-        const Grid g{s.nTheta, s.nPhi, s.nPhi >> 1, s.invNP};
-        const int N = g.nT * g.nP;
-        const Rsrc up = make_rsrc(s.state[parity][F_UPHI], N);
-        const Rsrc ut = make_rsrc(s.state[parity][F_UTHETA], N - g.nP);
-        const float2* __restrict__ in = reinterpret_cast<const float2*>(s.part[parity]);
-        float2* __restrict__ outp = reinterpret_cast<float2*>(s.part[parity ^ 1]);
-        const float invH = s.invH, R = s.radius, dt = s.dt;
-        const float cofTheta = dt / R;
-        const int end = tile.row0 + tile.rows;
-        for (int k = tile.row0 + (int)threadIdx.x; k < end; k += (int)blockDim.x) {
-            const float2 p = in[k];
-            // offset-shifted coordinates in cells: u_phi nodes sit at
-            // ((i - 1/2) h, (j + 1/2) h), u_theta nodes at (i h, (j + 1) h)
-            const float x = p.x * invH, y = p.y * invH;
-            const float uP = sample<K_VPHI>(up, g, 0, x + 0.5f, 0, y - 0.5f);
-            const float uT = sample<K_VTHETA>(ut, g, 0, x, 0, y - 1.f);
-            const float latRadius = R * sinf(p.y);
-            float th = p.y + uT * cofTheta;
-            float ph = p.x;
-            if (latRadius > 1e-7f) ph = p.x + uP * (dt / latRadius);
-            validate_coord(ph, th);
-            outp[k] = make_float2(ph, th);
-            flag_bad(s.status, !isfinite(ph) || !isfinite(th));
+    const int t = xcd_tile(ntiles);
+    if (t >= ntiles) return;
+    const Tile tile = tiles[t];
+    const SimDesc& s = sims[tile.sim];
+    const Grid g{s.nTheta, s.nPhi, s.nPhi >> 1, s.invNP};
+    const int N = g.nT * g.nP;
+    const Rsrc up = make_rsrc(s.state[parity][F_UPHI], N);
+    const Rsrc ut = make_rsrc(s.state[parity][F_UTHETA], N - g.nP);
+    const float2* __restrict__ in = reinterpret_cast<const float2*>(s.part[parity]);
+    float2* __restrict__ outp = reinterpret_cast<float2*>(s.part[parity ^ 1]);
+    const float invH = s.invH, R = s.radius, dt = s.dt;
+    const float cofTheta = dt / R;
+    const int end = tile.row0 + tile.rows;
+    // column of a cell index, as sample() folds it
+    auto column = [&](int ip) {
+        ip -= __mul24(g.nP, (int)floorf((float)ip * g.invNP));
+        ip += (ip < 0) ? g.nP : 0;
+        return ip - ((ip >= g.nP) ? g.nP : 0);
+    };
+    for (int k = tile.row0 + (int)threadIdx.x; k < end; k += (int)blockDim.x) {
+        const float2 p = in[k];
+        // offset-shifted coordinates in cells: u_phi nodes sit at
+        // ((i - 1/2) h, (j + 1/2) h), u_theta nodes at (i h, (j + 1) h);
+        // column() is exact for |x| up to some 2^22 only, and what lies outside
+        // the row takes the general path
+        const float x = p.x * invH, xP = fmaf(p.x, invH, 0.5f), yP = fmaf(p.y, invH, -0.5f);
+        float yT = p.y * invH;
+        asm("" : "+v"(yT));  // rounded before the shift
+        yT -= 1.f;
+        const int jP = cell_of(yP), jT = cell_of(yT);
+        float uP, uT;
+        const int iP = column(cell_of(xP)), iT = column(cell_of(x));
+        if (jP >= 1 && jP < g.nT - 2 && jT >= 1 && jT < g.nT - 3 && (unsigned)iP < (unsigned)g.nP &&
+            (unsigned)iT < (unsigned)g.nP) {
+            // both samples ordinary: sample()'s own case (less its last row,
+            // whose last pair would end past the field), the two columns of a
+            // row as one load, column 0 again where they wrap
+            const int oP = __mul24(jP, g.nP) + iP, oT = __mul24(jT, g.nP) + iT;
+            const float2 pA = ldf2(up, oP), pB = ldf2(up, oP + g.nP);
+            const float2 tA = ldf2(ut, oT), tB = ldf2(ut, oT + g.nP);
+            float pA1 = pA.y, pB1 = pB.y, tA1 = tA.y, tB1 = tB.y;
+            if (iP + 1 == g.nP) {
+                pA1 = ldf(up, oP + 1 - g.nP);
+                pB1 = ldf(up, oP + 1);
+            }
+            if (iT + 1 == g.nP) {
+                tA1 = ldf(ut, oT + 1 - g.nP);
+                tB1 = ldf(ut, oT + 1);
+            }
+            const float aP = frac_of(xP), aT = frac_of(x);
+            uP = lerpf(lerpf(pA.x, pA1, aP), lerpf(pB.x, pB1, aP), frac_of(yP));
+            uT = lerpf(lerpf(tA.x, tA1, aT), lerpf(tB.x, tB1, aT), frac_of(yT));
+        } else {
+            uP = sample<K_VPHI>(up, g, 0, xP, 0, yP);
+            uT = sample<K_VTHETA>(ut, g, 0, x, 0, yT);
         }
+        const float latRadius = R * sinf(p.y);
+        float th = p.y + uT * cofTheta;
+        float ph = p.x;
+        if (latRadius > 1e-7f) ph = p.x + uP * (dt / latRadius);
+        validate_coord(ph, th);
+        outp[k] = make_float2(ph, th);
+        flag_bad(s.status, !isfinite(ph) || !isfinite(th));
     }
 }
 
