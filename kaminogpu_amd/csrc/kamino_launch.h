@@ -23,8 +23,11 @@ constexpr int fft_row_stride(int M, bool padded) { return M + (padded ? M >> 4 :
 // a multiple of 4, at most half of every member's nPhi.
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                          int stride, int polarD, size_t ldsBytes, int gridCap, hipStream_t st);
-hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                            int gridCap, hipStream_t st);
+// the first `staged` tiles (at most kPartStaged particles each) sample the
+// velocities from LDS, ldsBytes of it; the others (at most 256) from memory
+constexpr int kPartStaged = 8192;
+hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int staged, size_t ldsBytes,
+                            int parity, int gridCap, hipStream_t st);
 // kernel: M where every row FFT of the launch has the same length M = 2^k >= 32
 // (FftPow2); else 1 when some rows span wavefronts, 0 when none does.
 hipError_t launch_div_fft(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,

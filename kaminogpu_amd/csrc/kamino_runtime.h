@@ -94,11 +94,11 @@ struct TileLayout {
     int nsims = 0, total = 0;
     int advOff = 0, nAdv = 0;
     int fftOff = 0, nFft = 0, nFft32 = 0, nFft64 = 0;  // FFT tiles (FP32-pressure ones first)
-    int partOff = 0, nPart = 0;
+    int partOff = 0, nPart = 0, nPartLds = 0;  // particle tiles (those that stage the fields first)
     int dftRowOff = 0, nDftRow = 0, dftOff = 0, nDft = 0;  // SIM_DFT rows and MFMA product tiles
     int ntri = 0;
     TriClass tri[12] = {};
-    size_t advLds = 0, fftLds = 0, fftLds64 = 0, divLds = 0;
+    size_t advLds = 0, partLds = 0, fftLds = 0, fftLds64 = 0, divLds = 0;
     int fftKernel = 0;  // the transform kernels' variant (launch_div_fft)
     int advStride = 0;  // staged row stride of the advection launch
     int polarD = 0;     // side columns of its polar tiles

@@ -629,6 +629,18 @@ static int shrink_until_busy(const Plan* plans, int n, int* rows, int minTiles, 
     }
 }
 
+static size_t part_lds(int nT) { return ((size_t)8 * nT * nT + 15) / 16 * 16; }
+// Particles sampled from LDS: a workgroup a CU stages both fields, 16 nTheta^2
+// bytes, instead of pulling 3.5 lines a particle through L1.  Steps measured
+// sampled from memory and from LDS: nTheta 80 with 400,000 particles 30.0 and
+// 29.9 us; 100 with 250,000 29.8 and 29.9, with 400,000 32.0 and 31.1, with
+// 1,000,000 39.9 and 34.5; 128 with 250,000 26.5 and 27.1, with 819,200 35.2
+// and 30.7; 64 with 400,000 25.4 and 25.7, 32 with 1,000,000 29.7 and 32.1 (L1
+// holds much of a small sphere).
+static bool staged_particles(const SimDesc& s) {
+    return s.nTheta >= 80 && part_lds(s.nTheta) <= kLdsMax && s.nPart >= 1536 * device_cus();
+}
+
 int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* out, int cap,
                TileLayout& L) {
     L = TileLayout();
@@ -801,8 +813,19 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     // 25.0 of 512, 23.3 of 256; with 819,200: 40.8, 38.8, 36.8, 36.2)
     constexpr int kPartTile = 256;
     L.partOff = cnt;
+    for (int s = 0; s < n; ++s) {
+        if (!staged_particles(sims[s])) continue;
+        // whole rounds of one workgroup a CU, in even runs
+        const int64_t N = sims[s].nPart, cus = device_cus();
+        const int64_t rounds = (N + cus * kPartStaged - 1) / (cus * kPartStaged);
+        const int run = (int)((N + cus * rounds * 64 - 1) / (cus * rounds * 64)) * 64;
+        for (int64_t k = 0; k < N; k += run) put(Tile{s, (int)k, (int)std::min<int64_t>(run, N - k), 0});
+        L.partLds = std::max(L.partLds, part_lds(sims[s].nTheta));
+    }
+    L.nPartLds = cnt - L.partOff;
     for (int s = 0; s < n; ++s)
-        for (int k = 0; k < sims[s].nPart; k += kPartTile) put(Tile{s, k, std::min(kPartTile, sims[s].nPart - k), 0});
+        for (int k = 0; k < sims[s].nPart && !staged_particles(sims[s]); k += kPartTile)
+            put(Tile{s, k, std::min(kPartTile, sims[s].nPart - k), 0});
     L.nPart = cnt - L.partOff;
     L.total = cnt;
     return cnt;
@@ -833,7 +856,7 @@ int launch_step(const SimDesc* dSims, const Tile* dTiles, const TileLayout& L, i
     if (phases & KAM_PHASE_ADVECT) {
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT], st));
         KAM_HIP(launch_advect(dSims, dTiles + L.advOff, L.nAdv, p, L.advStride, L.polarD, L.advLds, kGridCap, st));
-        KAM_HIP(launch_particles(dSims, dTiles + L.partOff, L.nPart, p, kGridCap, st));
+        KAM_HIP(launch_particles(dSims, dTiles + L.partOff, L.nPart, L.nPartLds, L.partLds, p, kGridCap, st));
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT + 1], st));
         p ^= 1;
     }

@@ -40,3 +40,26 @@ def test_particle_step_vs_oracle(nt, n):
     ref, amb = O.advect_particles(nt, 2 * nt, dt, up, ut, pos)
     if not amb.all():
         assert rel_pos(got, ref, amb) < TOL_POS
+
+
+@pytest.mark.parametrize("nt", [80, 125, 128, 135])
+@pytest.mark.parametrize("n", [1536 * 256, 600001, 8192 * 256 + 65])
+def test_staged_particles_equal_gathered(nt, n):
+    """Many particles are sampled from LDS; the same particles set a few at a
+    time are sampled from memory and land on the same positions to the bit."""
+    dt = 0.5 / nt
+    state = [np.ascontiguousarray(a, np.float32) for a in O.init_fields(nt, 2 * nt, 8, nt, 1)]
+    pos = positions(nt, n, nt)
+    pos[:4] = [[np.nan, 1.0], [1.0, np.inf], [1e30, 1.0], [-1e9, 0.5]]
+    with K.Sim(nt, dt) as s:
+        s.set_fields(*state)
+        s.set_particles(pos)
+        s.step_phases(K.PHASE_ADVECT)
+        got = s.get_particles()
+    part = 300000
+    for k in range(0, n, part):
+        with K.Sim(nt, dt) as s:
+            s.set_fields(*state)
+            s.set_particles(pos[k:k + part])
+            s.step_phases(K.PHASE_ADVECT)
+            np.testing.assert_array_equal(got[k:k + part], s.get_particles())
