@@ -1642,6 +1642,13 @@ __device__ __forceinline__ T shfl_grp(T v, int srcLaneInGroup, int laneBase) {
 // copy (parity ^ 1), K consecutive entries per lane, and skips the FP32
 // write-back.
 constexpr int kTriBatch = 4;  // float4 spectrum loads per thread in flight while staging
+// Lanes of 32 rows (nTheta > 1024) take their off-diagonals into registers,
+// through the LDS that the mode columns take next: 75 KB a workgroup instead of
+// 91, so a CU holds two, and the 512 workgroups of one 2048 x 4096 sphere run
+// at once, not in two rounds (24.9 -> 20.1 us; of 1500 x 3000, three spheres,
+// 74.2 -> 52.1).
+template <int KMAX, bool RESID, typename T>
+constexpr bool tri_tab_regs = KMAX == 32 && !RESID && std::is_same<T, float>::value;
 
 // A block is one dependent chain (stage, Thomas, log2 L reductions, back
 // substitution, write back) on few waves, so what bounds it on a single sphere
@@ -1659,12 +1666,13 @@ constexpr int kTriBatch = 4;  // float4 spectrum loads per thread in flight whil
 template <int L, int KMAX, bool RESID, typename T, bool FULL>
 __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, const Tile& tile,
                                             int parity, float2* zsp, double* csp, double* ssp,
-                                            float* fsp) {
+                                            float* fsp, float* fss) {
     // SF: the subtraction-free pivots of the FP32 elimination, from FP32 row
     // tables; the FP64 row terms are staged for the FP64 elimination and for
     // the residual report
     constexpr bool SF = std::is_same<T, float>::value;
     constexpr bool kStage64 = !SF || RESID;
+    constexpr bool kTabRegs = tri_tab_regs<KMAX, RESID, T>;
     constexpr int NR = KMAX * (L + 1);
     auto zs = [&](int gg, int k, int ll) -> float2& { return zsp[(gg * KMAX + k) * (L + 1) + ll]; };
     auto cs = [&](int k, int ll) -> double& { return csp[k * (L + 1) + ll]; };
@@ -1672,7 +1680,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
     // FP32 rows: sub-diagonal, super-diagonal (pole folds included), 1/sin^2
     auto fa = [&](int k, int ll) -> float& { return fsp[k * (L + 1) + ll]; };
     auto fc = [&](int k, int ll) -> float& { return fsp[NR + k * (L + 1) + ll]; };
-    auto fs = [&](int k, int ll) -> float& { return fsp[2 * NR + k * (L + 1) + ll]; };
+    auto fs = [&](int k, int ll) -> float& { return fss[k * (L + 1) + ll]; };
     const int tid = threadIdx.x;
     const int l = tid % L;               // lane within the mode group
     const int g = tid / L;               // mode within the block
@@ -1787,6 +1795,16 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
                 }
             }
         }
+        T ta[kTabRegs ? KMAX : 1], tc[kTabRegs ? KMAX : 1];
+        if constexpr (kTabRegs) {
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < KMAX; ++k) {
+                ta[k] = fa(k, l);
+                tc[k] = fc(k, l);
+            }
+            __syncthreads();  // the mode columns overwrite the tables
+        }
         for (int base = 0; base < nPairs; base += 256 * kTriBatch) {
             if (base > 0) load(base);
 #pragma unroll
@@ -1852,7 +1870,9 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
                     const float2 f = zs(g, k, l);
                     const T fr = (n == 0) ? T(0) : (T)f.x, fi = (T)f.y;
                     if constexpr (SF) {
-                        const T a = fa(k, l), c = fc(k, l), m = nnf * fs(k, l);
+                        const T a = kTabRegs ? ta[kTabRegs ? k : 0] : fa(k, l);
+                        const T c = kTabRegs ? tc[kTabRegs ? k : 0] : fc(k, l);
+                        const T m = nnf * fs(k, l);
                         const T sig = m + a * tau;
                         const T inv = rcpT(c + sig);
                         const T ep = (m + a * epPrev) * inv;
@@ -2062,23 +2082,25 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
 
 template <int L, int KMAX, bool RESID, typename T>
 __device__ __forceinline__ void tri_tile(const SimDesc* __restrict__ sims, const Tile& tile, int parity, float2* zsp,
-                                         double* csp, double* ssp, float* fsp) {
+                                         double* csp, double* ssp, float* fsp, float* fss) {
     if (tile.rows == 256 / L && sims[tile.sim].nTheta == L * KMAX)
-        tri_tile_as<L, KMAX, RESID, T, true>(sims, tile, parity, zsp, csp, ssp, fsp);
+        tri_tile_as<L, KMAX, RESID, T, true>(sims, tile, parity, zsp, csp, ssp, fsp, fss);
     else
-        tri_tile_as<L, KMAX, RESID, T, false>(sims, tile, parity, zsp, csp, ssp, fsp);
+        tri_tile_as<L, KMAX, RESID, T, false>(sims, tile, parity, zsp, csp, ssp, fsp, fss);
 }
 
 template <int L, int KMAX, bool RESID, typename T>
-__global__ __launch_bounds__(256) void k_tridiag(const SimDesc* __restrict__ sims,
+__global__ __launch_bounds__(256, (tri_tab_regs<KMAX, RESID, T>) ? 2 : 1) void k_tridiag(const SimDesc* __restrict__ sims,
                                                  const Tile* __restrict__ tiles, int ntiles, int parity) {
     __shared__ float2 zs[(256 / L) * KMAX * (L + 1)];
     constexpr bool SF = std::is_same<T, float>::value;
     constexpr int NR = KMAX * (L + 1);
     __shared__ double cs[(!SF || RESID) ? NR : 1], ss[(!SF || RESID) ? NR : 1];
-    __shared__ float fr[SF ? 3 * NR : 1];
+    constexpr bool kTabRegs = tri_tab_regs<KMAX, RESID, T>;
+    __shared__ float fr[!SF ? 1 : (kTabRegs ? NR : 3 * NR)];
     for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles)
-        tri_tile<L, KMAX, RESID, T>(sims, tiles[t], parity, zs, cs, ss, fr);
+        tri_tile<L, KMAX, RESID, T>(sims, tiles[t], parity, zs, cs, ss,
+                                    kTabRegs ? reinterpret_cast<float*>(zs) : fr, kTabRegs ? fr : fr + 2 * NR);
 }
 
 // Every class with K = 8 rows per lane in one launch: a tile carries its lanes
@@ -2096,10 +2118,10 @@ __global__ __launch_bounds__(256) void k_tridiag_mixed(const SimDesc* __restrict
     for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles) {
         const Tile tile = tiles[t];
         switch (tile.col0) {
-            case 8: tri_tile<8, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr); break;
-            case 16: tri_tile<16, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr); break;
-            case 32: tri_tile<32, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr); break;
-            default: tri_tile<64, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr); break;
+            case 8: tri_tile<8, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr, fr + 2 * K * 9); break;
+            case 16: tri_tile<16, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr, fr + 2 * K * 17); break;
+            case 32: tri_tile<32, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr, fr + 2 * K * 33); break;
+            default: tri_tile<64, K, RESID, T>(sims, tile, parity, zs, cs, ss, fr, fr + 2 * K * 65); break;
         }
     }
 }
