@@ -426,8 +426,6 @@ __device__ __forceinline__ unsigned wave_max(unsigned v) {
     v = dpp_max<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
     return dpp_max<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
-constexpr int kAdvWaves = 256 / 64;  // wavefronts of an advection workgroup
-
 // Displacement budgets of the fast path, in cells.  Node columns sit at
 // staged columns kEC-1 .. W+kEC and sample offsets lie within half a cell,
 // so phi departures below 2.5 cells keep the stencil in [0, W + 2 kEC); node
@@ -449,12 +447,13 @@ constexpr float kFastDPhi = 2.4f, kFastDTheta = 1.4f;
 // leaves the CU; the cubic roots reuse the staged block's LDS.
 // Flat item loops split an index into (row, column) with a magic multiply.
 // ---------------------------------------------------------------------------
-template <int SW>
-__global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims,
+template <int SW, int NW>
+__global__ __launch_bounds__(64 * NW) void k_advect(const SimDesc* __restrict__ sims,
                                                 const Tile* __restrict__ tiles, int ntiles,
                                                 int parity, int polarD) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    constexpr int nthr = kAdvWaves * 64;  // launch_advect's block size
+    constexpr int nthr = NW * 64;
+    constexpr bool kApart = NW > kAdvWaves;  // the advected block beside the rho plane, not over it
     const int tid = threadIdx.x;
     for (int t = xcd_tile(ntiles); t < ntiles; t = ntiles) {
         const Tile tile = tiles[t];
@@ -508,14 +507,14 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         const int W1 = W + 1, W2 = W + 2;
         const int uvN = geom ? (R + 1) * W2 + (R + 2) * W1 + 2 * W1 : 0;
         float* cofRow[3];
-        cofRow[0] = lds + (polar ? 3 * plane + uvN : 2 * plane + max(plane, uvN));
+        cofRow[0] = lds + (polar || kApart ? 3 * plane + uvN : 2 * plane + max(plane, uvN));
         cofRow[1] = cofRow[0] + (R + 2);
         cofRow[2] = cofRow[1] + (R + 2);
         // per wavefront: max |u_phi|, |u_theta| of its staged items and max
         // half phi coefficient of its node rows (float bits), after the
         // coefficients.  The kernel has no static LDS, so the dynamic block
         // starts at address 0 and LDS offsets fold into the instructions.
-        unsigned(*wmax)[kAdvWaves] = reinterpret_cast<unsigned(*)[kAdvWaves]>(cofRow[2] + (R + 2));
+        unsigned(*wmax)[NW] = reinterpret_cast<unsigned(*)[NW]>(cofRow[2] + (R + 2));
         unsigned mc = 0u;
         if (tid < R + 2) {  // node rows j0-1 .. j0+R, one per thread
             const int j = j0 - 1 + tid;
@@ -630,7 +629,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
 #pragma unroll
             for (int k = 0; k < 3; ++k)
 #pragma unroll
-                for (int w = 0; w < kAdvWaves; ++w) m[k] = max(m[k], wmax[k][w]);
+                for (int w = 0; w < NW; ++w) m[k] = max(m[k], wmax[k][w]);
             const float Up = __uint_as_float(m[0]), Ut = __uint_as_float(m[1]);
             const float hmax = __uint_as_float(m[2]);
             // a departure moves at most 2 h max|u| cells
@@ -657,6 +656,15 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         using KTheta = std::integral_constant<int, K_VTHETA>;
         using KRho = std::integral_constant<int, K_CENTERED>;
 
+        // A stride-SW launch holds widths up to SW - 2 kEC, and the column map
+        // serves exactly that width: the row step rmS is then a constant, and
+        // rm0 (a whole wavefront's tile row, kColW being a multiple of 64) is
+        // uniform over the wavefront, so the walks' trip counts are scalar.
+        constexpr int kColW = SW - 2 * kEC, rmS = nthr / kColW;
+        static_assert(kColW % 64 == 0 && nthr % kColW == 0, "a column map row is whole wavefronts");
+        const bool colMap = (W == kColW);
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
+
         // ---- a polar tile's backtraces, as tasks of 64 columns that the
         // wavefronts take in turn; the tile's edge columns form tasks of their
         // own (a task's lanes are nodes of one kind)
@@ -664,8 +672,9 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         const int vLo = max(j0 - 1, 0), vHi = min(j0 + R, nT - 2);
         const bool north = (j0 == 0), south = (uHi == nT - 1);
         // the rho nodes go first; in tiles clear of the poles their staged
-        // plane then holds U, V, A0, AL (polar tiles keep these apart)
-        float* U = lds + (polar ? 3 : 2) * plane;  // (R+1) x W2: u_phi*, columns c0-1 .. c0+W
+        // plane then holds U, V, A0, AL (polar tiles and wide workgroups keep
+        // these apart)
+        float* U = lds + (polar || kApart ? 3 : 2) * plane;  // (R+1) x W2: u_phi*, columns c0-1 .. c0+W
         float* V = U + (R + 1) * W2;               // (R+2) x W1: u_theta*, columns c0-1 .. c0+W-1
         float* A0 = V + __mul24(R + 2, W1);        // W1: u_theta* of row 0 at the antipodal columns
         float* AL = A0 + W1;                       // W1: u_theta* of row nT-2 at the antipodal columns
@@ -678,7 +687,6 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
             ps.rlo = rlo;
             ps.rows[K_VPHI] = ps.rows[K_CENTERED] = min(nT, js + SR) - rlo;
             ps.rows[K_VTHETA] = min(nT - 1, js + SR) - rlo;
-            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
             const int v0 = geom ? vLo : j0;
             const int nUr = geom ? uHi - uLo + 1 : R, nVr = geom ? vHi - vLo + 1 : min(R, nT - 1 - j0);
             const int nA = geom ? (north ? 1 : 0) + (south ? 1 : 0) : 0;
@@ -686,7 +694,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
             const int tR = R * nc, tU = nUr * nc, tV = (nVr + nA) * nc;
             const int tUe = geom ? (2 * nUr + 63) >> 6 : 0, tVe = geom ? (nVr + nA + 63) >> 6 : 0;
             bool bad = false;
-            for (int t = wave; t < tR + tU + tUe + tV + tVe; t += kAdvWaves) {
+            for (int t = wave; t < tR + tU + tUe + tV + tVe; t += NW) {
                 int k = t;
                 if (k < tR) {
                     const int r = k >> wide, c = ln + (wide ? (k & 1) << 6 : 0), j = j0 + r;
@@ -745,6 +753,27 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         } else if (!geom) {
             auto plain = [&](auto F) __attribute__((always_inline)) {
                 bool bad = false;
+                if (kApart && colMap) {  // a task: 64 columns of a row, one kind of node
+                    constexpr int nc = kColW / 64;
+                    const int tR = R * nc;
+                    for (int t = wave; t < 3 * tR; t += NW) {
+                        const int kind = t < tR ? K_CENTERED : (t < 2 * tR ? K_VPHI : K_VTHETA);
+                        const int k = t - (t < tR ? 0 : (t < 2 * tR ? tR : 2 * tR));
+                        const int r = k / nc, c = ln + ((k % nc) << 6), j = j0 + r;
+                        const int colB = (c0 + c) * 4, rowB = j * nP * 4;
+                        if (kind == K_CENTERED) {
+                            const float a = node(F, KRho{}, c, j, cofRow[0][r + 1]);
+                            stf(orhR, colB, rowB, a);
+                            bad |= !isfinite(a);
+                        } else if (kind == K_VPHI) {
+                            stf(oupR, colB, rowB, node(F, KPhi{}, c, j, cofRow[0][r + 1]));
+                        } else if (j < nT - 1) {
+                            stf(outR, colB, rowB, node(F, KTheta{}, c, j, cofRow[1][r + 1]));
+                        }
+                    }
+                    flag_bad(status, bad);
+                    return;
+                }
                 for (int idx = tid; idx < R * W; idx += nthr) {
                     const int r = (int)__umulhi((unsigned)idx, mW), c = idx - r * W;
                     const int j = j0 + r, o = j * nP + c0 + c;
@@ -775,17 +804,49 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
         // wavefront down.  Other widths split a flat item index; those loops end
         // at wavefront granularity, with no duplicated tail items (occupancy
         // hides the LDS latency).  The mapping never changes a value.
-        // A stride-SW launch holds widths up to SW - 2 kEC, and the column map
-        // serves exactly that width: the row step rmS is then a constant, and
-        // rm0 (a whole wavefront's tile row, kColW being a multiple of 64) is
-        // uniform over the wavefront, so the walks' trip counts are scalar.
-        constexpr int kColW = SW - 2 * kEC, rmS = nthr / kColW;
-        static_assert(kColW % 64 == 0 && nthr % kColW == 0, "a column map row is whole wavefronts");
-        const bool colMap = (W == kColW);
         const int cm = tid & (kColW - 1), rm0 = __builtin_amdgcn_readfirstlane(tid / kColW);
         const int colB = (c0 + cm) * 4;  // the lane's column in a row of the grid, in bytes
         const int nUr = uHi - uLo + 1, nVr = vHi - vLo + 1;
         auto advect_all = [&](auto F) __attribute__((always_inline)) {
+            if (kApart && colMap) {
+                // a task: 64 columns of a row, or the edge columns of 32 or 64
+                // rows, of one kind of node
+                constexpr int nc = kColW / 64;
+                const int tR = R * nc, tU = nUr * nc, tV = nVr * nc;
+                const int tUe = (2 * nUr + 63) >> 6, tVe = (nVr + 63) >> 6;
+                bool bad = false;
+                for (int t = wave; t < tR + tU + tUe + tV + tVe; t += NW) {
+                    int k = t;
+                    if (k < tR) {
+                        const int r = k / nc, c = ln + ((k % nc) << 6);
+                        const float a = node(F, KRho{}, c, j0 + r, cofRow[0][r + 1]);
+                        stf(orhR, (c0 + c) * 4, (j0 + r) * nP * 4, a);
+                        bad |= !isfinite(a);
+                        continue;
+                    }
+                    k -= tR;
+                    if (k < tU + tUe) {
+                        int r = k / nc, c = ln + ((k % nc) << 6);
+                        if (k >= tU) {  // columns -1 and W
+                            const int e = ((k - tU) << 6) + ln;
+                            r = e >> 1;
+                            c = (e & 1) ? W : -1;
+                        }
+                        if (r < nUr)
+                            U[__mul24(r, W2) + c + 1] = node(F, KPhi{}, c, uLo + r, cofRow[0][uLo + r - j0 + 1]);
+                        continue;
+                    }
+                    k -= tU + tUe;
+                    int r = k / nc, c = ln + ((k % nc) << 6);
+                    if (k >= tV) {  // column -1
+                        r = ((k - tV) << 6) + ln;
+                        c = -1;
+                    }
+                    if (r < nVr) V[__mul24(r, W1) + c + 1] = node(F, KTheta{}, c, vLo + r, cofRow[1][vLo + r - j0 + 1]);
+                }
+                flag_bad(status, bad);
+                return;
+            }
             if (colMap) {
                 const int dOfs = __mul24(rmS, SW);
                 int ofs = __mul24(j0 + rm0 - js, SW) + cm + kEC;
@@ -796,7 +857,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
                     bad |= !isfinite(a);
                 }
                 flag_bad(status, bad);
-                __syncthreads();  // the staged rho plane is dead from here on
+                if (!kApart) __syncthreads();  // the staged rho plane is dead from here on
                 ofs = __mul24(uLo + rm0 - js, SW) + cm + kEC;
                 float* u = U + __mul24(rm0, W2) + cm + 1;
                 for (int r = rm0; r < nUr; r += rmS, ofs += dOfs, u += __mul24(rmS, W2))
@@ -824,7 +885,7 @@ __global__ __launch_bounds__(256) void k_advect(const SimDesc* __restrict__ sims
                 bad |= !isfinite(a);
             }
             flag_bad(status, bad);
-            __syncthreads();  // the staged rho plane is dead from here on
+            if (!kApart) __syncthreads();  // the staged rho plane is dead from here on
             for (int idx = tid; idx < nU; idx += nthr) {
                 const int r = (int)__umulhi((unsigned)idx, mW2), c = idx - __mul24(r, W2) - 1, j = uLo + r;
                 U[idx] = node(F, KPhi{}, c, j, cofRow[0][j - j0 + 1]);
@@ -2301,17 +2362,19 @@ static inline int grid_for(int ntiles, int cap) {
 }
 
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                         int stride, int polarD, size_t ldsBytes, int gridCap, hipStream_t st) {
+                         int stride, int waves, int polarD, size_t ldsBytes, int gridCap, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    if (stride == adv_stride(64))
-        hipLaunchKernelGGL(k_advect<adv_stride(64)>, dim3(grid_for(ntiles, gridCap)), dim3(256),
-                           ldsBytes, st, sims, tiles, ntiles, parity, polarD);
-    else if (stride == adv_stride(128))
-        hipLaunchKernelGGL(k_advect<adv_stride(128)>, dim3(grid_for(ntiles, gridCap)), dim3(256),
-                           ldsBytes, st, sims, tiles, ntiles, parity, polarD);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+    const dim3 grid(grid_for(ntiles, gridCap)), block(64 * waves);
+#define KAM_ADVECT(SW, NW)                                                                                \
+    if (stride == (SW) && waves == (NW)) {                                                                \
+        hipLaunchKernelGGL((k_advect<SW, NW>), grid, block, ldsBytes, st, sims, tiles, ntiles, parity, polarD); \
+        return hipGetLastError();                                                                         \
+    }
+    KAM_ADVECT(adv_stride(64), kAdvWaves)
+    KAM_ADVECT(adv_stride(64), kAdvWavesWide)
+    KAM_ADVECT(adv_stride(128), kAdvWaves)
+#undef KAM_ADVECT
+    return hipErrorInvalidValue;
 }
 
 // Moves ranges with vector accesses (which also works where a caller captures
@@ -2463,9 +2526,10 @@ hipError_t configure_kernels(size_t bytes) {
 #define KAM_FNS(m)                                                                     \
     (const void*)k_div_fft<m>, (const void*)k_ifft_grad<float2, false, m>,             \
         (const void*)k_ifft_grad<double2, false, m>,
-    const void* fns[] = {KAM_FFT_POW2(KAM_FNS) KAM_FNS(0) KAM_FNS(1)(const void*) k_advect<adv_stride(64)>,
+    const void* fns[] = {KAM_FFT_POW2(KAM_FNS) KAM_FNS(0) KAM_FNS(1)(const void*) k_advect<adv_stride(64), kAdvWaves>,
+                         (const void*)k_advect<adv_stride(64), kAdvWavesWide>,
                          (const void*)k_particles_lds,
-                         (const void*)k_advect<adv_stride(128)>, (const void*)k_ifft_grad<float2, true, 1>,
+                         (const void*)k_advect<adv_stride(128), kAdvWaves>, (const void*)k_ifft_grad<float2, true, 1>,
                          (const void*)k_ifft_grad<double2, true, 1>};
 #undef KAM_FNS
     for (const void* fn : fns) {

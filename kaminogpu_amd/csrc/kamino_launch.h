@@ -21,8 +21,11 @@ constexpr int fft_row_stride(int M, bool padded) { return M + (padded ? M >> 4 :
 
 // polarD: columns that polar tiles stage on either side of theirs (PolarStage),
 // a multiple of 4, at most half of every member's nPhi.
+// waves: wavefronts of a workgroup, kAdvWaves or, at the narrower stride,
+// kAdvWavesWide.
+constexpr int kAdvWaves = 4, kAdvWavesWide = 8;
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
-                         int stride, int polarD, size_t ldsBytes, int gridCap, hipStream_t st);
+                         int stride, int waves, int polarD, size_t ldsBytes, int gridCap, hipStream_t st);
 // the first `staged` tiles (at most kPartStaged particles each) sample the
 // velocities from LDS, ldsBytes of it; the others (at most 256) from memory
 constexpr int kPartStaged = 8192;

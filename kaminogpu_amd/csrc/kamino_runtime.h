@@ -101,6 +101,7 @@ struct TileLayout {
     size_t advLds = 0, partLds = 0, fftLds = 0, fftLds64 = 0, divLds = 0;
     int fftKernel = 0;  // the transform kernels' variant (launch_div_fft)
     int advStride = 0;  // staged row stride of the advection launch
+    int advWaves = 0;   // wavefronts of its workgroups
     int polarD = 0;     // side columns of its polar tiles
 };
 

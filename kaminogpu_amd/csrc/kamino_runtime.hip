@@ -54,14 +54,16 @@ static int factor_m(int M, int* fac) {
 // (k_advect): the staged input block, plus with the geometric update the
 // advected u_phi and u_theta rows and the antipodal rows (the cubic roots
 // reuse the staged block)
-static size_t adv_lds(int R, int W, int SW, bool geometric) {
+static size_t adv_lds(int R, int W, int SW, bool geometric, int waves = kAdvWaves) {
     // three staged planes; with the geometric update the advected u_phi*,
     // u_theta* and antipodal rows go over the third (rho) plane once the rho
-    // nodes are done, spilling past it when larger; then three per-row
-    // coefficients of rows j0-1 .. j0+R and three maxima per wavefront
+    // nodes are done, spilling past it when larger (beside it in workgroups of
+    // more waves); then three per-row coefficients of rows j0-1 .. j0+R and
+    // three maxima per wavefront
     const size_t plane = (size_t)(R + 2 * kAdvHaloRows) * SW;
     const size_t uv = geometric ? (size_t)(R + 1) * (W + 2) + (R + 2) * (W + 1) + 2 * (W + 1) : 0;
-    return (2 * plane + std::max(plane, uv) + 3 * (size_t)(R + 2) + 3 * (256 / 64)) * sizeof(float);
+    const size_t third = waves > kAdvWaves ? plane + uv : std::max(plane, uv);
+    return (2 * plane + third + 3 * (size_t)(R + 2) + 3 * waves) * sizeof(float);
 }
 // Rows of a band starting within kAdvHaloRows + 1 rows of a pole, or ending
 // there (polar_rows: the bands next to the poles are that tall if R allows).
@@ -76,7 +78,7 @@ static size_t polar_lds(int nT, int R, int poleTile, int W, int D, bool geometri
     const int rows = std::min(nT, polar_bands(nT, R) ? std::min(kPoleRows, r + kAdvHaloRows) + kAdvHaloRows
                                                      : r + 2 * kAdvHaloRows);
     const size_t uv = geometric ? (size_t)(r + 1) * (W + 2) + (r + 2) * (W + 1) + 2 * (W + 1) : 0;
-    return ((size_t)3 * rows * 2 * (W + 2 * D) + uv + 3 * (size_t)(r + 2) + 3 * (256 / 64)) * sizeof(float);
+    return ((size_t)3 * rows * 2 * (W + 2 * D) + uv + 3 * (size_t)(r + 2) + 3 * kAdvWavesWide) * sizeof(float);
 }
 // The elementary radices and items per lane of each kind of FFT pass.
 struct Radices {
@@ -674,12 +676,26 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
                 set_tile_cols(sims[s], advCols[s]);
             }
     L.advStride = adv_stride(wide && !narrow ? kAdvMaxCols : kAdvMaxCols / 2);
+    // A launch of few cells, whose length is a tile's dependent phases one after
+    // the other, takes workgroups of eight waves, a tile a CU (four of them by
+    // LDS, whatever heights were set).  Steps of one sphere with four waves and
+    // two tiles a CU, and so: nTheta 32 20.2 and 19.7 us, 75 23.5 and 22.9,
+    // 192 25.6 and 24.5; but 256 22.0 and 22.6, 625 47.0 and 48.9.
+    int64_t cells = 0;
+    size_t apart = 0;
+    for (int s = 0; s < n; ++s) {
+        cells += (int64_t)plans[s].nT * plans[s].nP;
+        apart = std::max(apart, adv_lds(advRows[s], advCols[s], L.advStride, (sims[s].flags & SIM_GEOMETRIC) != 0,
+                                        kAdvWavesWide));
+    }
+    const bool small = cells <= 384 * (int64_t)device_cus() && apart <= 40 * 1024 && L.advStride == adv_stride(64);
+    L.advWaves = small ? kAdvWavesWide : kAdvWaves;
     // A launch of few tiles runs them all at once and lasts as long as its
     // slowest: the polar bands, whose samples take the pole rules, go out as
     // tiles of one row there (a 256 x 512 step 25.5 us with four-row ones, 24.4
     // with two, 23.7 with one; from 512 x 1024 on the same or, with few rows
     // left to the other tiles, 0.5 us slower).
-    const int advTiles = shrink_until_busy(plans, n, advRows, minTiles, advCols);
+    const int advTiles = shrink_until_busy(plans, n, advRows, small ? minTiles / 2 : minTiles, advCols);
     const bool few = advTiles <= 4 * device_cus();
     const int poleTile = few ? 1 : kPoleRows;
     shrink_until_busy(plans, n, fftRows, minTiles, nullptr);
@@ -705,7 +721,7 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
                 rows = std::min(R, p.nT - kPoleRows - j);
             for (int c = 0; c < p.nP; c += W) put(Tile{s, j, rows, std::min(c, p.nP - W)});
         }
-        L.advLds = std::max(L.advLds, adv_lds(advRows[s], W, L.advStride, (sims[s].flags & SIM_GEOMETRIC) != 0));
+        L.advLds = std::max(L.advLds, adv_lds(advRows[s], W, L.advStride, (sims[s].flags & SIM_GEOMETRIC) != 0, L.advWaves));
     }
     L.nAdv = cnt;
     // The polar tiles' side columns: what a flow of speed 1.25 moves in the row
@@ -855,7 +871,7 @@ int launch_step(const SimDesc* dSims, const Tile* dTiles, const TileLayout& L, i
     }
     if (phases & KAM_PHASE_ADVECT) {
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT], st));
-        KAM_HIP(launch_advect(dSims, dTiles + L.advOff, L.nAdv, p, L.advStride, L.polarD, L.advLds, kGridCap, st));
+        KAM_HIP(launch_advect(dSims, dTiles + L.advOff, L.nAdv, p, L.advStride, L.advWaves, L.polarD, L.advLds, kGridCap, st));
         KAM_HIP(launch_particles(dSims, dTiles + L.partOff, L.nPart, L.nPartLds, L.partLds, p, kGridCap, st));
         if (ev) KAM_HIP(hipEventRecord(ev[2 * KC_ADVECT + 1], st));
         p ^= 1;
