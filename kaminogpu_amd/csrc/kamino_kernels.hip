@@ -426,6 +426,7 @@ __device__ __forceinline__ unsigned wave_max(unsigned v) {
     v = dpp_max<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
     return dpp_max<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
+
 // Displacement budgets of the fast path, in cells.  Node columns sit at
 // staged columns kEC-1 .. W+kEC and sample offsets lie within half a cell,
 // so phi departures below 2.5 cells keep the stencil in [0, W + 2 kEC); node
@@ -446,6 +447,13 @@ constexpr float kFastDPhi = 2.4f, kFastDTheta = 1.4f;
 // (assignPhiKernel :517-534, assignThetaKernel :537-549) before anything
 // leaves the CU; the cubic roots reuse the staged block's LDS.
 // Flat item loops split an index into (row, column) with a magic multiply.
+//
+// Large launches are bound by vector instructions (324 a cell) and LDS reads:
+// 128 spheres of 256 x 512 take 156 us, of which issue is 137 and LDS 104.
+// Small ones last as long as a tile's phases in turn.  NW = 8 (plan_tiles):
+// the advected block lies beside the staged rho plane, no barrier parts the
+// three kinds of node, and wavefronts take rows of one kind in turn; a step of
+// one sphere 23.6 -> 22.8 us at nTheta 75, 25.7 -> 24.5 at 192.
 // ---------------------------------------------------------------------------
 template <int SW, int NW>
 __global__ __launch_bounds__(64 * NW) void k_advect(const SimDesc* __restrict__ sims,
@@ -1714,8 +1722,8 @@ constexpr bool tri_tab_regs = KMAX == 32 && !RESID && std::is_same<T, float>::va
 // A block is one dependent chain (stage, Thomas, log2 L reductions, back
 // substitution, write back) on few waves, so what bounds it on a single sphere
 // is its instruction count, about 5 cycles each per wave; large batches are
-// bound by the spectrum's 16 bytes per cell (268 MB in 29.9 us, 9 TB/s through
-// the caches, at 128 spheres of 256).  Hence no slot of a staging batch that no
+// bound by the spectrum's 8 bytes per cell (134 MB in 27 to 30 us, 4.5 to 5
+// TB/s, at 128 spheres of 256).  Hence no slot of a staging batch that no
 // thread needs, one reciprocal per reduction, shared by shuffle with both
 // neighbours, and no selects at the ends of a group.
 //

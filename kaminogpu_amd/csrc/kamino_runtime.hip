@@ -702,7 +702,7 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     // advection tiles, in batch order (tallest simulations first); the last
     // column tile of a row band overlaps its neighbour instead of running short.
     // A tile starting within kAdvHaloRows + 1 rows of a pole (or ending within
-    // them) samples with the checked sampler throughout, so the two polar bands
+    // them) is a polar one (PolarStage in k_advect), so the two polar bands
     // are exactly that tall when the tile height allows, and every band between
     // them can take the fast one; the last inner band may be shorter.
     L.advOff = 0;
