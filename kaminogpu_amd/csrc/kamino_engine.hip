@@ -870,13 +870,21 @@ int kam_autotune(int device, int n_theta, int batch, int steps, const char* cach
     uint64_t id;
     for (int b = 0; b < batch && rc == KAM_OK; ++b)
         rc = kam_engine_admit(e, &d, up.data(), ut.data(), rho.data(), (int64_t)1 << 40, &id);
-    // candidates: advection tiles, then FFT tile heights, each timed on its own kernels
-    const int rowsC[4] = {4, 8, 12, 16}, colsC[2] = {64, 128};
+    // candidates: advection tiles, then FFT tile heights, each timed on its own kernels.
+    // A batch of small spheres times alike with most of them, and the first
+    // ones timed read up to a third high while the clocks rise; so an untimed
+    // pass goes first, and a later candidate has to be 3% faster than the best
+    // so far, tall and narrow ones going first (ties had picked short or wide
+    // tiles at random, which cost a mixed batch of 64 spheres up to 9% of its
+    // step).
+    constexpr double kGain = 0.97;
+    const int rowsC[4] = {16, 12, 8, 4}, colsC[2] = {64, 128};
     const int fftMax = base.fftRows;
     const int fftC[3] = {fftMax, std::max(1, fftMax / 2), std::max(1, fftMax / 4)};
     double best[KC_COUNT] = {1e30, 1e30, 1e30, 1e30};
     int bestR = base.advRows, bestW = base.advCols, bestF = base.fftRows;
     double k[KC_COUNT];
+    if (rc == KAM_OK) rc = kam_engine_profile(e, 4 * steps, k);
     for (int ci = 0; ci < 2 && rc == KAM_OK; ++ci)
         for (int ri = 0; ri < 4 && rc == KAM_OK; ++ri) {
             if (colsC[ci] > nP) continue;
@@ -884,7 +892,7 @@ int kam_autotune(int device, int n_theta, int batch, int steps, const char* cach
             e->dirty = true;
             if ((rc = kam_engine_profile(e, 2, k)) != KAM_OK) break;
             if ((rc = kam_engine_profile(e, steps, k)) != KAM_OK) break;
-            if (k[KC_ADVECT] < best[KC_ADVECT]) {
+            if (k[KC_ADVECT] < kGain * best[KC_ADVECT]) {
                 best[KC_ADVECT] = k[KC_ADVECT];
                 bestR = rowsC[ri];
                 bestW = colsC[ci];
@@ -897,7 +905,7 @@ int kam_autotune(int device, int n_theta, int batch, int steps, const char* cach
         if ((rc = kam_engine_profile(e, 2, k)) != KAM_OK) break;
         if ((rc = kam_engine_profile(e, steps, k)) != KAM_OK) break;
         const double f = k[KC_DIVFFT] + k[KC_IFFT];
-        if (f < best[KC_DIVFFT] + best[KC_IFFT]) {
+        if (f < kGain * (best[KC_DIVFFT] + best[KC_IFFT])) {
             best[KC_DIVFFT] = k[KC_DIVFFT];
             best[KC_IFFT] = k[KC_IFFT];
             best[KC_TRI] = k[KC_TRI];

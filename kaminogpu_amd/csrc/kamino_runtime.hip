@@ -665,13 +665,15 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     // stride and with the largest member's LDS.  When members were tuned to
     // different widths, the wide ones (alone a launch too small to fill the
     // GPU) are restaged as narrow tiles of the same area, so that the narrow
-    // majority keeps its occupancy.  Tile shapes never change a value.
+    // majority keeps its occupancy; no taller than 16 rows by that, since one
+    // member's 32 x 64 tiles set the whole launch's LDS (64 uneven spheres: 35 us
+    // of advection for 31).  Tile shapes never change a value.
     bool narrow = false, wide = false;
     for (int s = 0; s < n; ++s) (advCols[s] > kAdvMaxCols / 2 ? wide : narrow) = true;
     if (narrow && wide)
         for (int s = 0; s < n; ++s)
             if (advCols[s] > kAdvMaxCols / 2) {
-                advRows[s] = std::min(2 * advRows[s], kAdvMaxRows);
+                advRows[s] = std::min(2 * advRows[s], std::max(advRows[s], 16));
                 advCols[s] = kAdvMaxCols / 2;
                 set_tile_cols(sims[s], advCols[s]);
             }
