@@ -24,7 +24,6 @@ namespace {
 constexpr size_t kScratchBytes = (size_t)KAM_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 16;
 constexpr int kMaxTiles = 4096;
-constexpr int kMaxTheta = 2048;  // the library's n_theta limit (host table staging)
 
 // One copy per device that loads the library.  In host code this name is a
 // stand-in, not a device address: host code uses the address that

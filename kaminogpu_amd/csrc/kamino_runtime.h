@@ -23,6 +23,8 @@ int set_err(int code, const char* fmt, ...);
             return ::kam::set_err(KAM_EHIP, "%s: %s", #call, hipGetErrorString(e_)); \
     } while (0)
 
+constexpr int kMaxTheta = 2048;  // the library's n_theta limit
+
 // Passes and lanes per row of the row FFT of M complex values.
 struct FftPlan {
     int nPass = 0, lanes = 0;

@@ -179,17 +179,14 @@ static void search_fft(int M, const int* fac, int nfac, FftPlan& best) {
     }
 }
 // The plan of M, searched for once (a rebuild of an engine's batch plans every
-// member; the search takes some 50 us).
+// member; the search takes some 50 us).  Static storage: the no-allocation step
+// plans its shape on every call and uses no heap.
 static std::mutex g_fft_mu;
-static std::map<int, FftPlan> g_fft;
+static FftPlan g_fft[kMaxTheta + 1];  // by M; no passes: not planned yet
 static void plan_fft(int M, const int* fac, int nfac, FftPlan& plan) {
     std::lock_guard<std::mutex> lk(g_fft_mu);
-    auto it = g_fft.find(M);
-    if (it == g_fft.end()) {
-        it = g_fft.emplace(M, FftPlan()).first;
-        search_fft(M, fac, nfac, it->second);
-    }
-    plan = it->second;
+    if (g_fft[M].nPass == 0) search_fft(M, fac, nfac, g_fft[M]);
+    plan = g_fft[M];
 }
 // LDS row stride of a transform row in complex values
 static int fft_stride(int M) { return fft_row_stride(M, (M & (M - 1)) == 0 && M >= 64); }
@@ -239,7 +236,7 @@ static TuneEntry tune_get(int nT) {
 int make_plan(int nT, int nP, Plan& p) {
     if (nT < 4) return set_err(KAM_EINVAL, "n_theta must be >= 4 (got %d)", nT);
     if (nP != 2 * nT) return set_err(KAM_EINVAL, "n_phi must equal 2*n_theta (got %d, %d)", nP, nT);
-    if (nT > 2048) return set_err(KAM_EINVAL, "n_theta must be <= 2048 (got %d)", nT);
+    if (nT > kMaxTheta) return set_err(KAM_EINVAL, "n_theta must be <= %d (got %d)", kMaxTheta, nT);
     p = Plan();
     p.nT = nT;
     p.nP = nP;

@@ -1,0 +1,78 @@
+"""CPU tests of the host side that plans a step (kaminogpu_amd/csrc/
+kamino_runtime.hip): a small C++ program linked with the library calls it, with
+no GPU call made."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+import kaminogpu_amd as K
+
+PKG = os.path.dirname(os.path.abspath(K.__file__))
+ROOT = os.path.dirname(PKG)
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+
+def run_cpp(tmp_path, source, *args):
+    """Builds `source` against the library and returns what it prints."""
+    K.lib()
+    src, exe = tmp_path / "main.cpp", tmp_path / "main"
+    src.write_text(source)
+    build = ["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
+             "-I", os.path.join(PKG, "csrc"), "-isystem", "/opt/rocm/include", "-o", str(exe), str(src),
+             "-L", PKG, "-lkamino", f"-Wl,-rpath,{PKG}", "-Wl,-rpath-link,/opt/rocm/lib"]
+    r = subprocess.run(build, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-4000:]
+    r = subprocess.run([str(exe), *args], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-2000:])
+    return r.stdout
+
+
+# Every heap allocation of the process goes through these; the no-allocation
+# step (kam_sim_step_noalloc) plans its shape and fills its tables on the host.
+COUNTED = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+
+#include "kamino.h"
+#include "kamino_runtime.h"
+
+static long g_count = 0;
+void* operator new(std::size_t n) {
+    ++g_count;
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+
+static float rowf[kam::RT_COUNT * 512], tw[4 * 512];
+static double rowd[kam::RD_COUNT * 512], tw64[4 * 512];
+
+int main() {
+    long plans = 0;
+    for (int pass = 0; pass < 2; ++pass)
+        for (int n = 4; n <= 512; ++n) {
+            int m = n;
+            for (int p : {2, 3, 5})
+                while (m % p == 0) m /= p;
+            if (m != 1) continue;
+            kam::Plan plan;
+            const long before = g_count;
+            if (kam::make_plan(n, 2 * n, plan) != KAM_OK) return 1;
+            if (pass) kam::compute_tables(n, 0.5 / n, 1.0, rowf, rowd, tw, tw64);
+            if (g_count != before) std::printf("n_theta %d: %ld allocations\n", n, g_count - before);
+            ++plans;
+        }
+    std::printf("%ld plans\n", plans);
+    return 0;
+}
+"""
+
+
+def test_planning_a_shape_uses_no_heap(tmp_path):
+    sizes = [n for n in range(4, 513) if (2 * 3 * 5) ** 9 % n == 0]  # 2^a 3^b 5^c
+    assert run_cpp(tmp_path, COUNTED) == f"{2 * len(sizes)} plans\n"
