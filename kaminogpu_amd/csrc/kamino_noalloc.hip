@@ -92,6 +92,12 @@ bool own_memory(const void* p, size_t bytes, int device) {
     return ok;
 }
 
+// Whether [a, a + na) and [b, b + nb) share a byte.
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + nb && q < p + na;
+}
+
 // Loads the descriptor, tiles and tables of this shape into the device's
 // scratch array (when it holds another shape), and waits for the upload.
 int load_shape(DevScratch& ds, const kam_sim_desc& d, const Plan& plan, hipStream_t st) {
@@ -192,13 +198,18 @@ extern "C" int kam_sim_step_noalloc(const kam_sim_desc* d, float* u_phi, float* 
     // and, without rho, the density read as zero.  One launch moves fields in
     // this device's memory; any others (host-mapped, another device's, or
     // past their allocation) go through the runtime's copies, which know how to
-    // reach them or refuse them.  One launch on either side of the steps in
-    // place of three copies and a clear before them and three copies after,
-    // each about 2 us of a call (one step of 32 x 64: 38.3 -> 29.7 us a call;
-    // eight of 256 x 512: 254 -> 246 us).
+    // reach them or refuse them.  So do fields that overlap (one buffer given
+    // twice): copied back one after the other, the later field's values stay,
+    // where the threads of one launch would race for them.  One launch on
+    // either side of the steps in place of three copies and a clear before them
+    // and three copies after, each about 2 us of a call (one step of 32 x 64:
+    // 38.3 -> 29.7 us a call; eight of 256 x 512: 254 -> 246 us).
     const bool direct = own_memory(u_phi, N * sizeof(float), d->device) &&
                         own_memory(u_theta, Nt * sizeof(float), d->device) &&
-                        (!rho || own_memory(rho, N * sizeof(float), d->device));
+                        (!rho || own_memory(rho, N * sizeof(float), d->device)) &&
+                        !overlap(u_phi, N * sizeof(float), u_theta, Nt * sizeof(float)) &&
+                        !(rho && overlap(rho, N * sizeof(float), u_phi, N * sizeof(float))) &&
+                        !(rho && overlap(rho, N * sizeof(float), u_theta, Nt * sizeof(float)));
     Ranges in = {{sd.state[0][F_UTHETA] + Nt, sd.state[1][F_UTHETA] + Nt, reinterpret_cast<float*>(sd.status),
                   sd.state[0][F_RHO], nullptr, nullptr},
                  {nullptr, nullptr, nullptr, rho, nullptr, nullptr},
