@@ -974,8 +974,12 @@ __global__ __launch_bounds__(64 * NW) void k_advect(const SimDesc* __restrict__ 
 //
 // What bounds it is the gathers, a cache line per lane and load, and below a
 // few thousand waves their latency.  So the two values a row of a sample needs
-// come as one load, and tiles are short (kPartTile).  A step of a 128 x 256
-// sphere with 100,000 particles, before and after: 35.9 and 23.3 us.
+// come as one load, and a particle has a thread: a step of a 128 x 256 sphere
+// with 100,000 takes 35.9 us with 2048 particles a workgroup, 28.4 with 1024,
+// 25.0 with 512, 23.3 with 256 (with 819,200: 40.8, 38.8, 36.8, 36.2).  A tile
+// keeps 2048 and serves eight workgroups, since the host plans, stages and
+// uploads every tile (16.8 million particles: 8192 tiles, 65,536 of 256; a step
+// of 256 x 512 with 1,000,000 takes 39.8 us either way).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void validate_coord(float& phi, float& theta) {
     constexpr double k2Pi = 6.28318530717958647692, kPiD = 3.14159265358979323846;
@@ -1054,12 +1058,15 @@ __device__ __forceinline__ float2 particle_move(const SimDesc& s, float2 p, floa
     return make_float2(ph, th);
 }
 
-__global__ __launch_bounds__(256) void k_particles(const SimDesc* __restrict__ sims,
+__global__ __launch_bounds__(kPartBlock) void k_particles(const SimDesc* __restrict__ sims,
                                                    const Tile* __restrict__ tiles, int ntiles,
                                                    int parity) {
-    const int t = xcd_tile(ntiles);
-    if (t >= ntiles) return;
-    const Tile tile = tiles[t];
+    constexpr int kShare = kPartTile / kPartBlock;  // workgroups of a tile
+    const int t = xcd_tile(ntiles * kShare);
+    if (t >= ntiles * kShare) return;
+    const Tile tile = tiles[t / kShare];
+    const int q = t % kShare * kPartBlock + (int)threadIdx.x;  // particle of the tile
+    if (q >= tile.rows) return;
     const SimDesc& s = sims[tile.sim];
     const Grid g{s.nTheta, s.nPhi, s.nPhi >> 1, s.invNP};
     const int N = g.nT * g.nP;
@@ -1068,8 +1075,7 @@ __global__ __launch_bounds__(256) void k_particles(const SimDesc* __restrict__ s
     const float2* __restrict__ in = reinterpret_cast<const float2*>(s.part[parity]);
     float2* __restrict__ outp = reinterpret_cast<float2*>(s.part[parity ^ 1]);
     const float invH = s.invH, cofTheta = s.dt / s.radius;
-    if ((int)threadIdx.x >= tile.rows) return;
-    const int k = tile.row0 + (int)threadIdx.x;
+    const int k = tile.row0 + q;
     const float2 p = in[k];
     const float uP = particle_uphi(up, g, p, invH), uT = particle_utheta(ut, g, p, invH);
     outp[k] = particle_move(s, p, uP, uT, cofTheta);
@@ -2420,8 +2426,8 @@ hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, 
     if (staged > 0)
         hipLaunchKernelGGL(k_particles_lds, dim3(staged), dim3(1024), ldsBytes, st, sims, tiles, staged, parity);
     if (ntiles > staged)
-        hipLaunchKernelGGL(k_particles, dim3(grid_for(ntiles - staged, gridCap)), dim3(256), 0, st, sims,
-                           tiles + staged, ntiles - staged, parity);
+        hipLaunchKernelGGL(k_particles, dim3(grid_for((ntiles - staged) * (kPartTile / kPartBlock), gridCap)),
+                           dim3(kPartBlock), 0, st, sims, tiles + staged, ntiles - staged, parity);
     return staged > 0 || ntiles > staged ? hipGetLastError() : hipSuccess;
 }
 

@@ -27,8 +27,9 @@ constexpr int kAdvWaves = 4, kAdvWavesWide = 8;
 hipError_t launch_advect(const SimDesc* sims, const Tile* tiles, int ntiles, int parity,
                          int stride, int waves, int polarD, size_t ldsBytes, int gridCap, hipStream_t st);
 // the first `staged` tiles (at most kPartStaged particles each) sample the
-// velocities from LDS, ldsBytes of it; the others (at most 256) from memory
-constexpr int kPartStaged = 8192;
+// velocities from LDS, ldsBytes of it; the others (at most kPartTile) from
+// memory, kPartTile / kPartBlock workgroups to a tile
+constexpr int kPartStaged = 8192, kPartTile = 2048, kPartBlock = 256;
 hipError_t launch_particles(const SimDesc* sims, const Tile* tiles, int ntiles, int staged, size_t ldsBytes,
                             int parity, int gridCap, hipStream_t st);
 // kernel: M where every row FFT of the launch has the same length M = 2^k >= 32

@@ -823,10 +823,7 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
             else
                 L.tri[L.ntri++] = TriClass{inMixed ? 0 : c[0], c[1], off, num, fp32 == 1};
         }
-    // particle tiles: runs of kPartTile particles, one a thread (a step of a
-    // 128 x 256 sphere with 100,000: 35.9 us in runs of 2048, 28.4 of 1024,
-    // 25.0 of 512, 23.3 of 256; with 819,200: 40.8, 38.8, 36.8, 36.2)
-    constexpr int kPartTile = 256;
+    // particle tiles: runs of kPartTile particles, or the staged ones' runs
     L.partOff = cnt;
     for (int s = 0; s < n; ++s) {
         if (!staged_particles(sims[s])) continue;

@@ -76,3 +76,55 @@ int main() {
 def test_planning_a_shape_uses_no_heap(tmp_path):
     sizes = [n for n in range(4, 513) if (2 * 3 * 5) ** 9 % n == 0]  # 2^a 3^b 5^c
     assert run_cpp(tmp_path, COUNTED) == f"{2 * len(sizes)} plans\n"
+
+
+# Tiles of one sphere's particles, from `plan_tiles` alone.
+PARTICLES = r"""
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "kamino_runtime.h"
+
+int main(int, char** argv) {
+    const int nT = std::atoi(argv[1]);
+    const long long n = std::atoll(argv[2]);
+    kam::Plan plan;
+    if (kam::make_plan(nT, 2 * nT, plan) != KAM_OK) return 1;
+    kam_sim_desc sd{};
+    sd.n_theta = nT;
+    sd.n_phi = 2 * nT;
+    sd.radius = 1.0;
+    sd.dt = 0.5 / nT;
+    sd.geometric = 1;
+    kam::SimDesc d;
+    kam::fill_desc(d, plan, kam::Tables(), sd, nullptr);
+    d.nPart = (int)n;
+    int rows[4];
+    kam::TileLayout L;
+    const int need = kam::plan_tiles(&d, &plan, 1, rows, nullptr, 0, L);
+    std::vector<kam::Tile> tiles((size_t)need);
+    kam::plan_tiles(&d, &plan, 1, rows, tiles.data(), need, L);
+    long long next = 0;  // the tiles cover every particle once, in order
+    int longest = 0;
+    for (int t = 0; t < L.nPart; ++t) {
+        const kam::Tile& tile = tiles[(size_t)(L.partOff + t)];
+        if (tile.row0 != next || tile.rows < 1) return 2;
+        next += tile.rows;
+        longest = std::max(longest, tile.rows);
+    }
+    if (next != n) return 3;
+    std::printf("%d %d %d\n", L.nPartLds, L.nPart, longest);
+    return 0;
+}
+"""
+
+
+def test_particle_tiles_are_few(tmp_path):
+    """A tile is 16 bytes to plan, stage and upload for at least 2048 particles."""
+    for nt, n in [(32, 1), (64, 2048), (64, 2049), (128, 100_000), (256, 1_000_000), (64, 1 << 26)]:
+        sub = tmp_path / f"{nt}_{n}"
+        sub.mkdir()
+        staged, tiles, longest = map(int, run_cpp(sub, PARTICLES, str(nt), str(n)).split())
+        assert staged == 0 and tiles == -(-n // 2048) and longest <= 2048, (nt, n, staged, tiles, longest)
