@@ -233,6 +233,18 @@ static TuneEntry tune_get(int nT) {
     return it == g_tune.end() ? TuneEntry{} : it->second;
 }
 
+// The FFT tile heights that a tuning entry or KAM_FFT_ROWS may name: 20480
+// complex values of LDS for the rows, a halo row, nPhi twiddles and a scratch
+// row per lane group, as the transform needed when the limit was set.  Callers
+// and caches hold entries up to it, so it stays; a tile then takes nTheta rows
+// at most, and what LDS holds of the padded rows (one less than the limit at
+// M = 256, never less elsewhere).
+static bool fft_rows_allowed(int rows, int M) {
+    int lanes = M >= 1024 ? 256 : 8;
+    while (lanes < 64 && 4 * lanes < M) lanes *= 2;
+    return ((size_t)rows + 3 + 256 / lanes) * M <= kLdsMax / 8;
+}
+
 int make_plan(int nT, int nP, Plan& p) {
     if (nT < 4) return set_err(KAM_EINVAL, "n_theta must be >= 4 (got %d)", nT);
     if (nP != 2 * nT) return set_err(KAM_EINVAL, "n_phi must equal 2*n_theta (got %d, %d)", nP, nT);
@@ -295,8 +307,9 @@ int adjust_plan(Plan& p, int advRows, int fftRows) {
         p.advLds = adv_lds(p.advRows, p.advCols, adv_stride(p.advCols), true);
     }
     if (fftRows > 0) {
-        if (fft_lds(fftRows, p.M) > 160 * 1024) return set_err(KAM_EINVAL, "FFT tile too tall");
+        if (!fft_rows_allowed(fftRows, p.M)) return set_err(KAM_EINVAL, "FFT tile too tall");
         p.fftRows = fftRows > p.nT ? p.nT : fftRows;
+        while (fft_lds(p.fftRows, p.M) > kLdsMax) --p.fftRows;
         p.fftLds = fft_lds(p.fftRows, p.M);
     }
     return KAM_OK;

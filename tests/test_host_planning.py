@@ -128,3 +128,21 @@ def test_particle_tiles_are_few(tmp_path):
         sub.mkdir()
         staged, tiles, longest = map(int, run_cpp(sub, PARTICLES, str(nt), str(n)).split())
         assert staged == 0 and tiles == -(-n // 2048) and longest <= 2048, (nt, n, staged, tiles, longest)
+
+
+def test_fft_heights_a_tuning_entry_may_name():
+    """Heights up to (20480 complex values of LDS) / M less three rows and a row
+    per lane group are taken, as many rows as the sphere has at most; taller
+    ones leave the default.  At 256 rows LDS holds one row less than the limit."""
+    for nt in [n for n in range(4, 2049) if (2 * 3 * 5) ** 11 % n == 0]:
+        K.tune_set(nt, 0, 0, 0)
+        default = K.tune_get(nt)[2]
+        lanes = next((g for g in (8, 16, 32) if 4 * g >= nt), 64) if nt < 1024 else 256
+        limit = 20480 // nt - 3 - 256 // lanes
+        try:
+            for rows in (1, 2, limit - 1, limit, limit + 1, 10 ** 6):
+                K.tune_set(nt, 0, 0, rows)
+                want = min(rows, nt, 72 if nt == 256 else nt) if rows <= limit else default
+                assert K.tune_get(nt)[2] == want, (nt, rows, limit)
+        finally:
+            K.tune_set(nt, 0, 0, 0)
