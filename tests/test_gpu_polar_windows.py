@@ -32,9 +32,9 @@ def fast_state(nt, dt):
 
 
 # The tolerance is the step's own.  A departure of x <= 100 cells carries FP32
-# errors of 6e-8 x from its rounding and 2e-7 x from its velocities, 3e-5 cells,
-# and the flow (m <= 8) changes by at most 8 pi / nt of itself per cell: below
-# 2e-6 at 512, less at smaller sizes, where x falls faster than 1 / nt grows.
+# errors of 6e-8 x from its rounding and 2e-7 x from its velocities, and the flow
+# (m <= 8) changes by at most 8 pi / nt of itself per cell: 2e-6 at 512, 4e-6 at
+# 16 (x <= 14).
 @pytest.mark.parametrize("nt", [16, 50, 75, 128, 256, 512])
 def test_departures_outside_the_windows_against_oracle(nt):
     dt = 0.5 / nt
