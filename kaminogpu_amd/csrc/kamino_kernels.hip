@@ -1563,8 +1563,28 @@ __global__ __launch_bounds__(kFftBlock) void k_div_fft(const SimDesc* __restrict
         // tile are read and not kept.  A lone wavefront pays ~5 cycles for
         // every instruction it issues, so slots that no thread of the block
         // needs (short tiles) are jumped over.
+        // Loads per point are what large launches wait for.  With 64 <= M <= 1024
+        // a slot's points of one wavefront lie in one row: its coefficients come
+        // as one load per wavefront and batch (coefficient c of slot q in lane
+        // 4c + q) instead of three per slot, and with M = 256 or 512 the slot
+        // kAbove back holds the point above, whose u_theta is this one's vn.
+        // us, before and after: 128 spheres of 256 rows 53.4 and 46.5, 43 of
+        // them 17.2 and 16.2, one 6.5 and 6.5; 32 of 512 57.4 and 52.2; 256 of
+        // 128 21.8 and 21.1; 8 of 1024 61.1 and 58.0.  At 2048, where a tile is
+        // one row, one sphere loses (32.7 and 33.2).
+        constexpr bool kWaveRows = MC >= 64 && MC <= 1024;
+        constexpr int kAbove = MC == 256 || MC == 512 ? MC / nthr : kDivBatch;
+        static_assert(RT_DIVN == RT_DIVS + 1 && RT_INVHS == RT_DIVS + 2 && kDivBatch == 4, "lane 4c + q");
         uint4 pv = make_uint4(0, 0, 0, 0);                         // the FFT passes, one per lane
         for (int base = 0; base < R * M; base += kDivBatch * nthr) {
+            float cof = 0.f;
+            if constexpr (kWaveRows) {  // lanes from 12 on read other entries or 0, not used
+                const int l = tid & 63, first = base + __builtin_amdgcn_readfirstlane(tid & ~63);
+                cof = ldf(rowR, (RT_DIVS + (l >> 2)) * nT + j0 + (first + (l & 3) * nthr) / M);
+            }
+            auto coefficient = [&](int c, int q) {
+                return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cof), 4 * c + q));
+            };
             float2 uw[kDivBatch], vn[kDivBatch], vs[kDivBatch];
             float ue1[kDivBatch], fs[kDivBatch], fn[kDivBatch], fi[kDivBatch];
             int rq[kDivBatch], kq[kDivBatch];
@@ -1577,11 +1597,13 @@ __global__ __launch_bounds__(kFftBlock) void k_div_fft(const SimDesc* __restrict
                 const int j = j0 + rq[q], oc = __mul24(j, nP) , i0 = 2 * kq[q], i2 = (i0 + 2 == nP) ? 0 : i0 + 2;
                 uw[q] = ldf2(upR, oc + i0);
                 ue1[q] = ldf(upR, oc + i2);
-                vn[q] = ldf2(utR, j > 0 ? oc - nP + i0 : -1);
+                if (q < kAbove) vn[q] = ldf2(utR, j > 0 ? oc - nP + i0 : -1);
                 vs[q] = ldf2(utR, oc + i0);
-                fs[q] = ldf(rowR, RT_DIVS * nT + j);
-                fn[q] = ldf(rowR, RT_DIVN * nT + j);
-                fi[q] = ldf(rowR, RT_INVHS * nT + j);
+                if constexpr (!kWaveRows) {
+                    fs[q] = ldf(rowR, RT_DIVS * nT + j);
+                    fn[q] = ldf(rowR, RT_DIVN * nT + j);
+                    fi[q] = ldf(rowR, RT_INVHS * nT + j);
+                }
             }
             // the twiddles are staged while the first points are in flight
             if (base == 0 && MC <= 1) pv = load_passes(s, tid);
@@ -1589,6 +1611,12 @@ __global__ __launch_bounds__(kFftBlock) void k_div_fft(const SimDesc* __restrict
 #pragma unroll
             for (int q = 0; q < kDivBatch; ++q) {
                 if (base + q * nthr >= R * M) break;
+                if constexpr (kWaveRows) {
+                    fs[q] = coefficient(0, q);
+                    fn[q] = coefficient(1, q);
+                    fi[q] = coefficient(2, q);
+                }
+                if (q >= kAbove) vn[q] = vs[q >= kAbove ? q - kAbove : 0];
                 if (rq[q] < R) {
                     const float d0 = (fs[q] * vs[q].x - fn[q] * vn[q].x) + fi[q] * (uw[q].y - uw[q].x);
                     const float d1 = (fs[q] * vs[q].y - fn[q] * vn[q].y) + fi[q] * (ue1[q] - uw[q].y);
