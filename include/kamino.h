@@ -354,12 +354,13 @@ int kam_tune_get(int n_theta, int *adv_rows, int *adv_cols, int *fft_rows);
 int kam_tune_set_transform(int n_theta, int transform);
 int kam_tune_get_transform(int n_theta, int *transform);
 
-/* Times candidate shapes on `batch` synthetic simulations of n_theta (steps
- * timed steps each): advection tiles, FFT tile heights, then the row FFT
- * against the MFMA DFT (n_theta <= 1024).  Records the fastest with
- * kam_tune_set and kam_tune_set_transform, appends a line
+/* Times candidate shapes on `batch` synthetic simulations of n_theta (five
+ * rounds over all of them, steps timed steps each): advection tiles, FFT tile
+ * heights, then the row FFT against the MFMA DFT (n_theta <= 1024).  Records,
+ * with kam_tune_set and kam_tune_set_transform, the default shapes or ones
+ * that are at least 4% faster in the median of the rounds, appends a line
  * "gfx950 n_theta batch adv_rows adv_cols fft_rows adv_ms fft_ms transform"
- * to cache_path (may be NULL), and returns the best per-kernel times in
+ * to cache_path (may be NULL), and returns the picks' mean per-kernel times in
  * kernel_ms[4] (advection, div+transform, tridiagonal, inverse
  * transform+gradient). */
 int kam_autotune(int device, int n_theta, int batch, int steps, const char *cache_path,

@@ -158,8 +158,8 @@ def tune_get_transform(n_theta):
 
 
 def autotune(n_theta, batch, steps=10, cache_path=None, device=0):
-    """Times candidate tile shapes on the device and keeps the fastest;
-    returns the best per-kernel times (ms)."""
+    """Times candidate tile shapes on the device and records the default ones or
+    clearly faster ones (kam_autotune); returns their per-kernel times (ms)."""
     k = (C.c_double * 4)()
     check(lib().kam_autotune(int(device), int(n_theta), int(batch), int(steps),
                              cache_path.encode() if cache_path else None, k))

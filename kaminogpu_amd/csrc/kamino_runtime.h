@@ -56,6 +56,11 @@ int tune_set(int nTheta, int advRows, int advCols, int fftRows);
 // Records the phi transform for n_theta (KAM_TRANSFORM_*; -1 = default FFT).
 int tune_set_transform(int nTheta, int transform);
 
+// The autotuner's choice among `shapes` shapes from their times in each round
+// (ms[round * shapes + shape]): shape 0, or one that is clearly faster.
+constexpr int kMaxRounds = 5;
+int pick_shape(const double* ms, int rounds, int shapes);
+
 // Sets or clears SIM_DFT on a simulation's descriptor from its plan and
 // precision, acquiring the shape's DFT matrices when needed (cached per
 // device and nPhi for the life of the process).

@@ -1,10 +1,12 @@
 """CPU tests of the host side that plans a step (kaminogpu_amd/csrc/
 kamino_runtime.hip): a small C++ program linked with the library calls it, with
 no GPU call made."""
+import math
 import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 import kaminogpu_amd as K
@@ -128,6 +130,50 @@ def test_particle_tiles_are_few(tmp_path):
         sub.mkdir()
         staged, tiles, longest = map(int, run_cpp(sub, PARTICLES, str(nt), str(n)).split())
         assert staged == 0 and tiles == -(-n // 2048) and longest <= 2048, (nt, n, staged, tiles, longest)
+
+
+# The autotuner's choice; arguments: rounds, then the times of each round.
+PICK = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "kamino_runtime.h"
+
+int main(int argc, char** argv) {
+    const int rounds = std::atoi(argv[1]);
+    std::vector<double> ms;
+    for (int k = 2; k < argc; ++k) ms.push_back(std::atof(argv[k]));
+    std::printf("%d\n", kam::pick_shape(ms.data(), rounds, (int)ms.size() / rounds));
+    return 0;
+}
+"""
+
+
+def test_autotuner_keeps_the_default_among_equals(tmp_path):
+    """Clocks that rise through the timings make later shapes look faster, and
+    equal shapes differ by some percent: neither moves the choice, nor does one
+    round that runs off.  A shape that is clearly faster does, of several the
+    fastest, or the first of those that time alike."""
+    rng = np.random.default_rng(3)
+
+    def pick(name, rel, noise=0.02, drift=0.0):
+        ms = np.empty((5, len(rel)))
+        for t, i in enumerate(np.ndindex(ms.shape)):
+            ms[i] = rel[i[1]] * (1 + drift * math.exp(-t / 4)) * (1 + noise * rng.uniform(-1, 1))
+        sub = tmp_path / name
+        sub.mkdir()
+        return int(run_cpp(sub, PICK, "5", *(f"{x:.6f}" for x in ms.ravel())))
+
+    for k in range(6):
+        assert pick(f"equal{k}", [1.0] * 9, drift=0.3) == 0
+    assert pick("faster", [1.0, 1.02, 0.9, 0.85, 0.99], drift=0.3) == 3
+    assert pick("alike", [1.0, 1.02, 0.90, 0.895, 0.89], noise=0.005) == 2
+    assert pick("slower", [1.0, 1.2, 1.1]) == 0
+    sub = tmp_path / "once"
+    sub.mkdir()
+    assert int(run_cpp(sub, PICK, "3", *"1 0.99 0.8 1 0.98 0.8 1.5 0.98 0.85".split())) == 2
+    assert int(run_cpp(sub, PICK, "3", *"1 0.99 1 0.98 1.5 0.98".split())) == 0
 
 
 def test_fft_heights_a_tuning_entry_may_name():
