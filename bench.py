@@ -133,7 +133,7 @@ GROUPS = 3  # set from --groups
 def tune(K, nt, batch, cache):
     """Tile shapes for n_theta: from the cache when it holds them, else timed on
     the device (kam_autotune) and appended to the cache.  Returns the tiles and
-    the best per-kernel times (None when loaded)."""
+    their per-kernel times (None when loaded)."""
     if cache and os.path.exists(cache) and not TUNED:
         TUNED.update(K.tune_load(cache))
     ms = None
@@ -142,7 +142,7 @@ def tune(K, nt, batch, cache):
         TUNED.add(nt)
     tiles = dict(zip(["adv_rows", "adv_cols", "fft_rows"], K.tune_get(nt)))
     # the phi transform the autotuner picked for this size: the row FFT or the MFMA DFT
-    tiles["transform"] = {K.TRANSFORM_DFT: "dft_mfma", K.TRANSFORM_FFT8: "fft_w8"}.get(K.tune_get_transform(nt), "fft")
+    tiles["transform"] = "dft_mfma" if K.tune_get_transform(nt) == K.TRANSFORM_DFT else "fft"
     return tiles, ms
 
 

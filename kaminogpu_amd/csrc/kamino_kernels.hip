@@ -1177,10 +1177,6 @@ __device__ __forceinline__ void lds_step(unsigned& a, int bytes) {
 __device__ __forceinline__ float2 mkc(float x, float y) { return make_float2(x, y); }
 __device__ __forceinline__ double2 mkc(double x, double y) { return make_double2(x, y); }
 template <typename C>
-__device__ __forceinline__ C cmul(C a, C b) {
-    return mkc(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-template <typename C>
 __device__ __forceinline__ C cadd(C a, C b) { return mkc(a.x + b.x, a.y + b.y); }
 template <typename C>
 __device__ __forceinline__ C csub(C a, C b) { return mkc(a.x - b.x, a.y - b.y); }

@@ -42,7 +42,7 @@ struct Plan {
     int triK = 0;      // template row capacity per lane
     size_t advLds = 0; // bytes of LDS of an advection tile (geometric on)
     size_t fftLds = 0; // bytes of LDS of an FFT tile (forward or inverse)
-    int transform = 0; // KAM_TRANSFORM_FFT, _FFT8, or _DFT (FP32-pressure simulations)
+    int transform = 0; // KAM_TRANSFORM_FFT (or its other name, _FFT8), or _DFT (FP32-pressure simulations)
 };
 
 // Validates a shape and fills its plan; returns KAM_OK or KAM_EINVAL.

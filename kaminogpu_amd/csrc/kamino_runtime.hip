@@ -65,8 +65,9 @@ static size_t adv_lds(int R, int W, int SW, bool geometric, int waves = kAdvWave
     const size_t third = waves > kAdvWaves ? plane + uv : std::max(plane, uv);
     return (2 * plane + third + 3 * (size_t)(R + 2) + 3 * waves) * sizeof(float);
 }
-// Rows of a band starting within kAdvHaloRows + 1 rows of a pole, or ending
-// there (polar_rows: the bands next to the poles are that tall if R allows).
+// Tiles starting within this many rows of a pole, or ending there, are polar
+// (PolarStage in k_advect); plan_tiles gives the poles bands of that height where
+// the tile height R allows it.
 constexpr int kPoleRows = kAdvHaloRows + 1;
 static bool polar_bands(int nT, int R) { return R >= kPoleRows && nT > 2 * kPoleRows; }
 // LDS of the polar tiles (k_advect, PolarStage): three planes of the rows they
@@ -283,7 +284,7 @@ int make_plan(int nT, int nP, Plan& p) {
     const TuneEntry te = tune_get(nT);
     // the MFMA DFT holds nPhi x nPhi matrices: offered up to n_theta = 1024
     if (te.transform == KAM_TRANSFORM_DFT && nT <= 1024) p.transform = KAM_TRANSFORM_DFT;
-    if (te.transform == KAM_TRANSFORM_FFT8) p.transform = KAM_TRANSFORM_FFT8;
+    if (te.transform == KAM_TRANSFORM_FFT8) p.transform = KAM_TRANSFORM_FFT8;  // runs as FFT; kam_tune_get_transform reports it
     if (te.advCols >= 8 && te.advCols <= kAdvMaxCols) p.advCols = te.advCols < nP ? te.advCols : nP;
     if (te.advRows > 0 || te.fftRows > 0) adjust_plan(p, te.advRows, te.fftRows);
     if (const char* v = std::getenv("KAM_ADV_COLS")) {
