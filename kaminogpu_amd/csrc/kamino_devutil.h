@@ -51,10 +51,6 @@ __device__ __forceinline__ void stf4(Rsrc r, int elem, float4 v) {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, elem * 4, 0, 0);
 }
-__device__ __forceinline__ void std2(Rsrc r, int elem, double2 v) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, elem * 16, 0, 0);
-}
 __device__ __forceinline__ float lerpf(float a, float b, float t) { return fmaf(t, b - a, a); }
 
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.

@@ -1762,6 +1762,10 @@ constexpr bool tri_tab_regs = KMAX == 32 && !RESID && std::is_same<T, float>::va
 // split into (lane, row) by shifts and pairs by constants.  A step of one
 // sphere, before these cuts and after: 23.8 -> 21.8 us at nTheta 256,
 // 62.3 -> 59.8 at 1024, 175 -> 167 at 2048; of 405, never full, 33.4 -> 33.3.
+// The guarded FP64 form stages its tables before the spectrum and stores x
+// through a pointer: with the spectrum's loads held across the tables, and with
+// range-checked stores, 20 spheres of 450 rows take 40.2 us for 35.8, 32 of 405
+// 51.7 for 47.4 (in the constant form both ways time alike).
 template <int L, int KMAX, bool RESID, typename T, bool FULL>
 __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, const Tile& tile,
                                             int parity, float2* zsp, double* csp, double* ssp,
@@ -1789,7 +1793,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
         const SimDesc& s = sims[tile.sim];
         const int nT = FULL ? L * KMAX : s.nTheta, Ms = FULL ? nT : s.M;
         const bool p64 = !SF;  // the FP64 elimination serves the FP64 pressure alone
-        const Rsrc spec64R = make_rsrc(s.state[parity ^ 1][0], p64 ? 4 * Ms * nT : 0);
+        double2* __restrict__ spec64 = reinterpret_cast<double2*>(s.state[parity ^ 1][0]);
         const bool active = FULL || g < tile.rows;
         const int n = tile.row0 + (active ? g : 0);
         const int rows = FULL ? 256 / L : tile.rows;  // the tile's modes
@@ -1832,8 +1836,10 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
             }
         };
         // staging: a thread's loads of a batch all go out before its first LDS
-        // write, the first batch's before the tables' too; reads past the
-        // tables or the spectrum return 0 and are not kept
+        // write, the first batch's before the tables' too (but for the guarded
+        // FP64 form); reads past the tables or the spectrum return 0 and are
+        // not kept
+        constexpr bool kEarly = SF || FULL;
         float4 v[kTriBatch];
         auto load = [&](int base) {
 #pragma unroll
@@ -1845,7 +1851,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
                 v[q] = ldf4(specR, p < nPairs ? 2 * a : -1);  // pairs past the tile read as 0, unused
             }
         };
-        load(0);
+        if constexpr (kEarly) load(0);
         if constexpr (kStage64) {
             const Rsrc rowR = make_rsrc(reinterpret_cast<const float*>(s.rowd), 2 * RD_COUNT * nT);
             for (int base = 0; base < nT; base += 4 * 256) {
@@ -1905,7 +1911,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
             __syncthreads();  // the mode columns overwrite the tables
         }
         for (int base = 0; base < nPairs; base += 256 * kTriBatch) {
-            if (base > 0) load(base);
+            if (!kEarly || base > 0) load(base);
 #pragma unroll
             for (int q = 0; q < kTriBatch; ++q) {
                 if (base + 256 * q >= nPairs) break;
@@ -2151,7 +2157,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
         for (int k = 0; k < KMAX; ++k) {
             if (k < cnt) {
                 if constexpr (!SF)
-                    std2(spec64R, n * nT + r0 + k, make_double2((n == 0) ? 0.0 : (double)xr[k], (double)xi[k]));
+                    spec64[(size_t)n * nT + r0 + k] = make_double2((n == 0) ? 0.0 : (double)xr[k], (double)xi[k]);
                 else
                     zs(g, k, l) = make_float2((n == 0) ? 0.f : (float)xr[k], (float)xi[k]);
             }
