@@ -31,10 +31,16 @@ struct FftPlan {
     FftPass pass[kFftMaxPass + 1] = {};
 };
 
+// What a size needs computed once: filled on its first plan, never changed.
+struct SizePlan {
+    FftPlan fft;
+    double sinPole;  // sin(h / 2), of the rows next to the poles
+};
+
 // Launch geometry of one simulation shape.
 struct Plan {
     int nT = 0, nP = 0, M = 0;
-    FftPlan fft;
+    const SizePlan* size = nullptr;
     int advRows = 0;   // rows per advection tile
     int advCols = 0;   // columns per advection tile
     int fftRows = 0;   // rows per FFT tile

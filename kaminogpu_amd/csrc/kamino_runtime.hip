@@ -3,6 +3,7 @@
 #include "kamino_runtime.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -179,15 +180,24 @@ static void search_fft(int M, const int* fac, int nfac, FftPlan& best) {
         }
     }
 }
-// The plan of M, searched for once (a rebuild of an engine's batch plans every
-// member; the search takes some 50 us).  Static storage: the no-allocation step
-// plans its shape on every call and uses no heap.
-static std::mutex g_fft_mu;
-static FftPlan g_fft[kMaxTheta + 1];  // by M; no passes: not planned yet
-static void plan_fft(int M, const int* fac, int nfac, FftPlan& plan) {
-    std::lock_guard<std::mutex> lk(g_fft_mu);
-    if (g_fft[M].nPass == 0) search_fft(M, fac, nfac, g_fft[M]);
-    plan = g_fft[M];
+// A size's own plan (M = nTheta), made on first use; the FFT search takes some
+// 50 us.  Plans point to it: a rebuild of an engine's batch plans every member
+// again, and a lock, a copy of the passes and a sine for each of 4096 had added a
+// sixth to its 1.6 ms.  Static storage: the no-allocation step plans its shape
+// on every call and uses no heap.
+static std::mutex g_size_mu;
+static SizePlan g_size[kMaxTheta + 1];
+static std::atomic<bool> g_sized[kMaxTheta + 1];
+static const SizePlan* size_plan(int M, const int* fac, int nfac) {
+    if (!g_sized[M].load(std::memory_order_acquire)) {
+        std::lock_guard<std::mutex> lk(g_size_mu);
+        if (!g_sized[M].load(std::memory_order_relaxed)) {
+            search_fft(M, fac, nfac, g_size[M].fft);
+            g_size[M].sinPole = std::sin(0.5 * (kPi / M));
+            g_sized[M].store(true, std::memory_order_release);
+        }
+    }
+    return &g_size[M];
 }
 // LDS row stride of a transform row in complex values
 static int fft_stride(int M) { return fft_row_stride(M, (M & (M - 1)) == 0 && M >= 64); }
@@ -265,7 +275,7 @@ int make_plan(int nT, int nP, Plan& p) {
     // mixed batches compact.
     p.advCols = nP < 64 ? nP : 64;
     p.advRows = nT < 128 ? (nT < 8 ? nT : 8) : 16;
-    plan_fft(p.M, fac, nfac, p.fft);
+    p.size = size_plan(p.M, fac, nfac);
     // FFT tile (the inverse adds a halo row): about four points per thread of
     // the forward transform.  Measured, us per step (FFT rows): 128 spheres of
     // 256 x 512 300 (2), 294 (4), 299 (8); 256 of 128 x 256 154 (4), 152 (8);
@@ -370,9 +380,8 @@ void compute_tables(int nT, double dt, double radius, float* rowf, double* rowd,
     for (int n = 0; n < M; ++n) w(n, tw64 + 2 * n);
     // then the passes' twiddles: of each pass those of its first radix, then
     // of its second (row_pass), for j = 0 .. Ls - 1 in a row
-    FftPlan pl;
     int fac[12] = {0};
-    plan_fft(M, fac, factor_m(M, fac), pl);
+    const FftPlan& pl = size_plan(M, fac, factor_m(M, fac))->fft;
     double* t = tw64 + 2 * M;
     for (int p = 0; p < pl.nPass; ++p) {
         const Radices r = kRadices[pl.pass[p].kind];
@@ -559,10 +568,10 @@ void fill_desc(SimDesc& d, const Plan& p, const Tables& t, const kam_sim_desc& s
     d.rowd = t.rowd;
     d.twN = t.twN;
     d.twN64 = t.twN64;
-    std::memcpy(d.pass, p.fft.pass, sizeof d.pass);
+    std::memcpy(d.pass, p.size->fft.pass, sizeof d.pass);
     d.passKinds = 0;
-    for (int k = 0; k < p.fft.nPass; ++k) d.passKinds |= 1u << p.fft.pass[k].kind;
-    d.fftShift = __builtin_ctz((unsigned)p.fft.lanes);
+    for (int k = 0; k < p.size->fft.nPass; ++k) d.passKinds |= 1u << p.size->fft.pass[k].kind;
+    d.fftShift = __builtin_ctz((unsigned)p.size->fft.lanes);
     d.advRows = p.advRows;
     d.fftRows = p.fftRows;
     d.magicP = (unsigned)((((uint64_t)1 << 32) + (uint64_t)p.nP - 1) / (uint64_t)p.nP);
@@ -744,8 +753,7 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
     const size_t room = few ? 40 * 1024 : std::max(L.advLds, (size_t)kLdsMax / 7);
     int most = 4;
     for (int s = 0; s < n; ++s) {
-        const double h = kPi / plans[s].nT;
-        const double cells = 1.25 * sims[s].cofTheta / std::sin(0.5 * h) + 3.0;
+        const double cells = 1.25 * sims[s].cofTheta / plans[s].size->sinPole + 3.0;
         most = std::max(most, (int)std::min(cells, 64.0));
     }
     for (int s = 0; s < n; ++s) most = std::min(most, plans[s].nP / 2);
@@ -781,7 +789,7 @@ int plan_tiles(SimDesc* sims, const Plan* plans, int n, int* rowScratch, Tile* o
             L.fftLds = std::max(L.fftLds, fft_lds(R, p.M));
             L.divLds = std::max(L.divLds, div_lds(R, p.M));
             commonM = (commonM < 0 || commonM == p.M) ? p.M : 0;
-            wideRows = wideRows || p.fft.lanes > 64;
+            wideRows = wideRows || p.size->fft.lanes > 64;
             if (p64) L.fftLds64 = std::max(L.fftLds64, fft_lds(R, p.M, true));
         }
     L.fftKernel = (commonM >= 32 && (commonM & (commonM - 1)) == 0) ? commonM : (wideRows ? 1 : 0);
@@ -915,17 +923,20 @@ int DeviceBatch::build(const std::vector<SimDesc>& simsIn, const std::vector<Pla
     const int n = (int)plans.size();
     std::vector<SimDesc> sims(simsIn);
     std::vector<int> rows(3 * (size_t)n + 1);
-    const int need = plan_tiles(sims.data(), plans.data(), n, rows.data(), nullptr, 0, lay_);
-    hTiles_.resize((size_t)need);
-    plan_tiles(sims.data(), plans.data(), n, rows.data(), hTiles_.data(), need, lay_);
+    // into the list of the last build; again where that is too short
+    int need = plan_tiles(sims.data(), plans.data(), n, rows.data(), hTiles_.data(), (int)hTiles_.size(), lay_);
+    if ((size_t)need > hTiles_.size()) {
+        hTiles_.resize((size_t)need);
+        need = plan_tiles(sims.data(), plans.data(), n, rows.data(), hTiles_.data(), need, lay_);
+    }
     cur_ ^= 1;
-    int rc = reserve(sims.size(), hTiles_.size(), st);
+    int rc = reserve(sims.size(), (size_t)need, st);
     if (rc != KAM_OK) return rc;
     // this staging buffer is free once its last upload, two rebuilds back,
     // has landed; the copies are queued behind the steps already launched
     KAM_HIP(hipEventSynchronize(uploaded_[cur_]));
     char* stage = static_cast<char*>(hStage_[cur_]);
-    const size_t sb = sims.size() * sizeof(SimDesc), tb = hTiles_.size() * sizeof(Tile);
+    const size_t sb = sims.size() * sizeof(SimDesc), tb = (size_t)need * sizeof(Tile);
     std::memcpy(stage, sims.data(), sb);
     std::memcpy(stage + capSims_ * sizeof(SimDesc), hTiles_.data(), tb);
     static_assert(sizeof(SimDesc) % 16 == 0 && sizeof(Tile) % 4 == 0, "moved in 4- or 16-byte values");
