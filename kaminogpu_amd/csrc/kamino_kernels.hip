@@ -1762,10 +1762,11 @@ constexpr bool tri_tab_regs = KMAX == 32 && !RESID && std::is_same<T, float>::va
 // split into (lane, row) by shifts and pairs by constants.  A step of one
 // sphere, before these cuts and after: 23.8 -> 21.8 us at nTheta 256,
 // 62.3 -> 59.8 at 1024, 175 -> 167 at 2048; of 405, never full, 33.4 -> 33.3.
-// The guarded FP64 form stages its tables before the spectrum and stores x
-// through a pointer: with the spectrum's loads held across the tables, and with
-// range-checked stores, 20 spheres of 450 rows take 40.2 us for 35.8, 32 of 405
-// 51.7 for 47.4 (in the constant form both ways time alike).
+// In FP64 the spectrum's loads follow the tables' (which return in order, so the
+// tables' LDS writes do not wait for them), and x is stored through a pointer:
+// with the loads first and range-checked stores, which the constant form bears,
+// the guarded one took 40.2 us for 33.9 at 20 spheres of 450 rows and 51.8 for
+// 45.6 at 32 of 405.
 template <int L, int KMAX, bool RESID, typename T, bool FULL>
 __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, const Tile& tile,
                                             int parity, float2* zsp, double* csp, double* ssp,
@@ -1836,10 +1837,9 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
             }
         };
         // staging: a thread's loads of a batch all go out before its first LDS
-        // write, the first batch's before the tables' too (but for the guarded
-        // FP64 form); reads past the tables or the spectrum return 0 and are
-        // not kept
-        constexpr bool kEarly = SF || FULL;
+        // write, the first batch's before the tables' or, in FP64, after them
+        // and before their writes; reads past the tables or the spectrum return
+        // 0 and are not kept
         float4 v[kTriBatch];
         auto load = [&](int base) {
 #pragma unroll
@@ -1851,7 +1851,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
                 v[q] = ldf4(specR, p < nPairs ? 2 * a : -1);  // pairs past the tile read as 0, unused
             }
         };
-        if constexpr (kEarly) load(0);
+        if constexpr (SF) load(0);
         if constexpr (kStage64) {
             const Rsrc rowR = make_rsrc(reinterpret_cast<const float*>(s.rowd), 2 * RD_COUNT * nT);
             for (int base = 0; base < nT; base += 4 * 256) {
@@ -1863,6 +1863,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
                     c[q] = ldd(rowR, RD_COT2H * nT + i0 + q * 256);
                     v[q] = ldd(rowR, RD_INVSIN2 * nT + i0 + q * 256);
                 }
+                if (!SF && base == 0) load(0);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     if (base + q * 256 >= nT) break;
@@ -1911,7 +1912,7 @@ __device__ __forceinline__ void tri_tile_as(const SimDesc* __restrict__ sims, co
             __syncthreads();  // the mode columns overwrite the tables
         }
         for (int base = 0; base < nPairs; base += 256 * kTriBatch) {
-            if (!kEarly || base > 0) load(base);
+            if (base > 0) load(base);
 #pragma unroll
             for (int q = 0; q < kTriBatch; ++q) {
                 if (base + 256 * q >= nPairs) break;
