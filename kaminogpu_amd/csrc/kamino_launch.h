@@ -67,9 +67,10 @@ constexpr int kDftTileRows = 64, kDftTileCols = 128, kDftChunk = 32;
 // launch; the kernel reads and writes them, so they are this device's memory or
 // pinned host memory.  A runtime copy between pinned and device memory goes to a
 // copy engine and back, 10 us and more in the stream for a few kilobytes: with
-// an engine's tables and finished fields moved by this kernel, 48 steps of 64
-// spheres of 32 to 256 rows with eight retirements take 3.5 to 4.2 ms instead of
-// 5.1.  (A copy stream beside the engine's for the finished fields: the same.)
+// an engine's tables and finished fields moved by this kernel, 40 steps of 96
+// spheres of 32 to 512 rows with twelve retirements take 8.4 ms instead of 9.2
+// (48 steps of 64 spheres of 32 to 256 rows with eight: 4.0 to 4.6 and 4.4 to
+// 4.8).  A copy stream beside the engine's for the finished fields: the same.
 constexpr int kMaxRanges = 6;
 struct Ranges {
     void* dst[kMaxRanges];
