@@ -24,7 +24,7 @@ def run_cpp(tmp_path, source, *args):
     src.write_text(source)
     build = ["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
              "-I", os.path.join(PKG, "csrc"), "-isystem", "/opt/rocm/include", "-o", str(exe), str(src),
-             "-L", PKG, "-lkamino", f"-Wl,-rpath,{PKG}", "-Wl,-rpath-link,/opt/rocm/lib"]
+             "-pthread", "-L", PKG, "-lkamino", f"-Wl,-rpath,{PKG}", "-Wl,-rpath-link,/opt/rocm/lib"]
     r = subprocess.run(build, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-4000:]
     r = subprocess.run([str(exe), *args], capture_output=True, text=True, timeout=300)
@@ -78,6 +78,54 @@ int main() {
 def test_planning_a_shape_uses_no_heap(tmp_path):
     sizes = [n for n in range(4, 513) if (2 * 3 * 5) ** 9 % n == 0]  # 2^a 3^b 5^c
     assert run_cpp(tmp_path, COUNTED) == f"{2 * len(sizes)} plans\n"
+
+
+# Eight threads plan every size at once, each in its own order.
+THREADS = r"""
+#include <atomic>
+#include <cstdio>
+#include <thread>
+#include <vector>
+
+#include "kamino_runtime.h"
+
+int main() {
+    std::vector<int> sizes;
+    for (int n = 4; n <= kam::kMaxTheta; ++n) {
+        int m = n;
+        for (int p : {2, 3, 5})
+            while (m % p == 0) m /= p;
+        if (m == 1) sizes.push_back(n);
+    }
+    std::atomic<int> ready{0}, bad{0};
+    std::vector<std::thread> threads;
+    for (int t = 0; t < 8; ++t)
+        threads.emplace_back([&, t] {
+            ++ready;
+            while (ready < 8) {}
+            for (size_t k = 0; k < sizes.size(); ++k) {
+                const int n = sizes[t & 1 ? sizes.size() - 1 - k : k];
+                kam::Plan p;
+                if (kam::make_plan(n, 2 * n, p) != KAM_OK) {
+                    ++bad;
+                    continue;
+                }
+                // complete: the passes' radices multiply to M (their items, to M / R)
+                const kam::FftPlan& f = p.size->fft;
+                long left = n;
+                for (int q = 0; q < f.nPass; ++q) left /= n / f.pass[q].nb;
+                if (left != 1 || f.lanes < 8 || !(p.size->sinPole > 0.0)) ++bad;
+            }
+        });
+    for (auto& t : threads) t.join();
+    std::printf("%zu sizes, %d bad\n", sizes.size(), bad.load());
+    return 0;
+}
+"""
+
+
+def test_planning_from_several_threads(tmp_path):
+    assert run_cpp(tmp_path, THREADS) == "107 sizes, 0 bad\n"
 
 
 # Tiles of one sphere's particles, from `plan_tiles` alone.
